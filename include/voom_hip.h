@@ -117,6 +117,27 @@ int voom_paged_gqa_combine(const int32_t* ctx_lens, void* out, float* lse_out,
                            int num_kv_heads, int head_dim, int page_tokens, int max_pages,
                            int num_splits, hipStream_t stream);
 
+/* Causal GQA attention of a window of query tokens over paged K/V.
+ *
+ * The multi-token branch of the reference's attention (explicit mask k_pos <=
+ * q_pos, runtime/layer_runner.py:166-177): the window's tokens are the newest
+ * of their sequences, query t sees the first seq_len - window + t + 1 tokens.
+ *
+ *   q          [batch, num_q_heads, window, head_dim] bf16 (already rotated)
+ *   out        [batch, window, num_q_heads, head_dim] bf16
+ *   seq_len    tokens of every sequence, the window included; all of them in
+ *              the block table [batch, max_pages]
+ *   workspace  voom_paged_gqa_prefill_workspace_bytes(...) bytes (may be 0:
+ *              then NULL is accepted)
+ * Same pools, heads, head_dim and page_tokens as voom_paged_gqa_decode. */
+size_t voom_paged_gqa_prefill_workspace_bytes(int batch, int num_q_heads, int num_kv_heads,
+                                              int head_dim, int window, int seq_len);
+int voom_paged_gqa_prefill(const void* q, const void* k_pool, const void* v_pool,
+                           const int32_t* block_table, void* out, void* workspace,
+                           size_t ws_bytes, int batch, int num_q_heads, int num_kv_heads,
+                           int head_dim, int page_tokens, int max_pages, int num_slots,
+                           int window, int seq_len, float scale, hipStream_t stream);
+
 /* Merge two attention states over disjoint key sets (log-sum-exp combine):
  * out = (o_a*e^{lse_a} + o_b*e^{lse_b}) / (e^{lse_a} + e^{lse_b}).
  * o_a/o_b/out [rows, head_dim] bf16, lse_* [rows] fp32; lse_out may be NULL.

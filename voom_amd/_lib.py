@@ -37,6 +37,10 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
                                         c_int, c_int, c_int, c_int, c_float, c_int, _P]),
     "voom_paged_gqa_combine": (c_int, [_P, _P, _P, _P, c_size_t, c_int, c_int, c_int, c_int,
                                        c_int, c_int, c_int, _P]),
+    "voom_paged_gqa_prefill_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int,
+                                                          c_int]),
+    "voom_paged_gqa_prefill": (c_int, [_P, _P, _P, _P, _P, _P, c_size_t, c_int, c_int, c_int,
+                                       c_int, c_int, c_int, c_int, c_int, c_int, c_float, _P]),
     "voom_merge_attn_states": (c_int, [_P, _P, _P, _P, _P, _P, c_int, c_int, _P]),
     "voom_fold_attn_state": (c_int, [_P, _P, _P, _P, c_int, c_int, c_int, _P]),
     "voom_mla_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),

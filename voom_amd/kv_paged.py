@@ -11,7 +11,7 @@ introspection its tests use, and adds the explicit verbs of the paged path:
   attend(layer, q, scale)  fused paged decode attention (HIP kernel); spilled
                            pages are reloaded on a side stream while the
                            resident pages are attended, then LSE-merged
-  attend_prefill(layer, q) causal attention of a prompt through the same kernel
+  attend_prefill(layer, q) causal attention of a prompt through the paged prefill kernel
   append_latent / update_latent / attend_mla
                            the absorbed-MLA latent cache (runtime/glm.py:265-330)
   spill(pages)             byte-plane split on the GPU -> D2H into the arena
@@ -1972,11 +1972,10 @@ class PagedKVCache:
         the queries of positions S-L .. S-1, whose K/V were just appended.
 
         The reference masks a multi-token window explicitly (k_pos <= q_pos,
-        runtime/layer_runner.py:166-177).  Here every query row becomes its own
-        entry of one paged decode call -- the same block-table row, with the
-        context cut at its own position + 1 -- so a prompt runs through the
-        paged kernel in one launch per 1024 query rows.  Spilled pages of the
-        layer are made resident first.
+        runtime/layer_runner.py:166-177).  Here the whole window runs through
+        the paged prefill kernel in one launch; a single token through the
+        decode kernel, which streams its K/V with every wavefront of the chip.
+        Spilled pages of the layer are made resident first.
         """
         self._require_kind(layer, "kv")
         B, NQ, L, D = q.shape
@@ -1989,18 +1988,19 @@ class PagedKVCache:
         if spilled:
             self.reload(spilled)
         pool = self._pool(layer)
-        rows_q = q.permute(0, 2, 1, 3).reshape(B * L, NQ, D).contiguous()
-        table = self._tables[layer].repeat_interleave(L, dim=0)
-        ctx = (torch.arange(S - L + 1, S + 1, dtype=torch.int32, device=self.device)
-               .repeat(B))
-        out = torch.empty_like(rows_q)
-        step = 1024  # rows per launch (the kernel's batch limit)
-        for r0 in range(0, B * L, step):
-            r1 = min(B * L, r0 + step)
-            out[r0:r1] = ops.paged_gqa_decode(rows_q[r0:r1], pool.k, pool.v,
-                                              table[r0:r1].contiguous(), ctx[r0:r1].contiguous(),
-                                              scale=scale)
-        return out.reshape(B, L, NQ, D).permute(0, 2, 1, 3)
+        table = self._tables[layer][:B]
+        q = q.contiguous()
+        if q.data_ptr() % 16:
+            q = q.clone()  # the kernels load 16 bytes per lane
+        if B == 0 or L == 0:
+            out = torch.empty((B, L, NQ, D), dtype=q.dtype, device=q.device)
+        elif L == 1 and B <= 1024:  # the decode kernel's batch limit
+            ctx = torch.full((B,), S, dtype=torch.int32, device=self.device)
+            out = ops.paged_gqa_decode(q.reshape(B, NQ, D), pool.k, pool.v, table, ctx,
+                                       scale=scale).reshape(B, L, NQ, D)
+        else:
+            out = ops.paged_gqa_prefill(q, pool.k, pool.v, table, S, scale=scale)
+        return out.permute(0, 2, 1, 3)
 
     def attend_mla(self, layer: int, q_nope: torch.Tensor, q_rope: torch.Tensor,
                    w_uk, w_uv_t, scale: float,

@@ -282,6 +282,41 @@ def paged_gqa_combine(ctx_lens: torch.Tensor, out: torch.Tensor, ws: torch.Tenso
     return out
 
 
+def paged_gqa_prefill(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
+                      block_table: torch.Tensor, seq_len: int, *,
+                      scale: float | None = None) -> torch.Tensor:
+    """Causal attention of a window of query tokens over paged K/V, one launch
+    (two where the window is split over keys).
+
+    q [B, NQ, L, D] bf16 holds the queries of each sequence's newest L of
+    ``seq_len`` tokens; block_table [B, max_pages] int32.  Returns [B, L, NQ, D].
+    """
+    _require(q.dim() == 4, "q must be [B, NQ, L, D]")
+    dev = _require_device(q, k_pool, v_pool, block_table)
+    B, NQ, L, D = q.shape
+    _require(k_pool.dim() == 4, "k_pool must be [slots, NKV, PT, D]")
+    slots, NKV, PT, Dk = k_pool.shape
+    _require(Dk == D, f"k_pool head_dim {Dk} != q head_dim {D}")
+    _check_v_pool(v_pool, slots, NKV, D, PT)
+    _require(q.dtype == k_pool.dtype == v_pool.dtype == torch.bfloat16,
+             "q and pools must be bfloat16")
+    _require(block_table.dtype == torch.int32 and block_table.dim() == 2
+             and block_table.shape[0] == B, "block_table must be int32 [B, max_pages]")
+    _require(NQ % NKV == 0, "num_q_heads must be a multiple of num_kv_heads")
+    if _BOUNDS_CHECKS:
+        check_block_table(block_table, torch.full((B,), seq_len, dtype=torch.int32, device=dev),
+                          slots, PT)
+    out = torch.empty((B, L, NQ, D), dtype=torch.bfloat16, device=dev)
+    # key-split partials: allocated per call, so calls on several streams or
+    # threads never share them
+    need = int(_lib.lib().voom_paged_gqa_prefill_workspace_bytes(B, NQ, NKV, D, L, seq_len))
+    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+    _lib.call("voom_paged_gqa_prefill", _ptr(q), _ptr(k_pool), _ptr(v_pool), _ptr(block_table),
+              _ptr(out), _ptr(ws), need, B, NQ, NKV, D, PT, block_table.shape[1], slots, L,
+              int(seq_len), float(D ** -0.5 if scale is None else scale), _stream(None))
+    return out
+
+
 def merge_attn_states(o_a: torch.Tensor, lse_a: torch.Tensor, o_b: torch.Tensor,
                       lse_b: torch.Tensor, *, stream: torch.cuda.Stream | None = None):
     """Combine two attention results over disjoint key sets (LSE merge)."""
