@@ -1,0 +1,148 @@
+"""GPU parity of position-free attention with many (query, head) columns -- the
+staged window kernels -- against fp64 attention over keys rotated as the entry
+point rotates them, and against the same call made one query at a time.
+
+Bars, relative L2 over the output: fp16 8e-4 (its own rounding is at most 2^-12 /
+sqrt(3) = 1.4e-4 per value and the rotated keys carry one fp16 rounding that can
+fall the other way than fp64's, 2^-11 of a key now and then; P is kept to 22
+bits), bf16 4e-3 (output and softmax weights rounded to bf16, 1.1e-3 each).
+"""
+import pytest
+import torch
+
+from voom_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+REL = {torch.float16: 8e-4, torch.bfloat16: 4e-3}
+
+
+def inputs(B, NQ, NKV, TQ, D, BLOCK, TK, dtype, seed, order="window", table_dtype=torch.float32):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    blocks = -(-TK // BLOCK)
+    P = max(1, blocks + 3)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda").to(dtype)  # noqa: E731
+    q = (2 * torch.randn((B, NQ, TQ, D), generator=g, device="cuda")).to(dtype)
+    table = torch.randint(0, P, (blocks,), generator=g, device="cuda", dtype=torch.int32)
+    kpos = torch.arange(TK, dtype=torch.int32, device="cuda")
+    qpos = torch.arange(TK - TQ, TK, dtype=torch.int32, device="cuda").clamp(min=0)
+    if order == "scattered":  # selected tokens anywhere, keys in any order
+        qpos = torch.randint(0, TK, (TQ,), generator=g, device="cuda", dtype=torch.int32)
+        kpos = kpos[torch.randperm(TK, generator=g, device="cuda")]
+    elif order == "all":
+        qpos = torch.full((TQ,), TK + 7, dtype=torch.int32, device="cuda")
+    elif order == "none":
+        kpos = kpos + 9
+        qpos = torch.full((TQ,), 3, dtype=torch.int32, device="cuda")
+    cos, sin = ops.rope_cache(TK + 16, D, 1e4, device="cuda")
+    return (q, rnd(P, NKV, BLOCK, D), rnd(P, NKV, BLOCK, D), table, kpos, qpos,
+            cos.to(table_dtype), sin.to(table_dtype))
+
+
+def reference(q, kp, vp, table, kpos, qpos, cos, sin, scale):
+    B, NQ, TQ, D = q.shape
+    _, NKV, BLOCK, _ = kp.shape
+    TK, half = kpos.numel(), D // 2
+    k = kp[table.long()].permute(1, 0, 2, 3).reshape(NKV, -1, D)[:, :TK].double()
+    v = vp[table.long()].permute(1, 0, 2, 3).reshape(NKV, -1, D)[:, :TK].double()
+    c, s = cos[kpos.long()].double(), sin[kpos.long()].double()
+    a, b = k[..., :half], k[..., half:]
+    k = torch.cat([a * c - b * s, b * c + a * s], -1).to(q.dtype).double()
+    hidden = kpos[None, :] > qpos[:, None]
+    G = NQ // NKV
+    out = torch.empty((B, NQ, TQ, D), dtype=torch.float64, device=q.device)
+    for h in range(NQ):
+        for b in range(B):
+            x = (q[b, h].double() @ k[h // G].t().contiguous() * scale).masked_fill(
+                hidden, -float("inf"))
+            w = torch.softmax(x, -1).nan_to_num(0.0)  # no visible key: zeros
+            out[b, h] = w @ v[h // G]
+    return out
+
+
+def check(got, ref, dtype):
+    torch.cuda.synchronize()
+    assert got.dtype == dtype and torch.isfinite(got).all()
+    rel = ((got.double() - ref).norm() / ref.norm().clamp(min=1e-30)).item()
+    assert rel <= REL[dtype], rel
+    row = ((got.double() - ref).norm(dim=-1) / ref.norm(dim=-1).clamp(min=1e-2)).max().item()
+    assert row <= 6 * REL[dtype], row
+
+
+def staged_from(B, NQ, NKV, D, TK):
+    """The fewest queries that take the staged route (window_pays in
+    position_free.hip): 56 columns plus one per 2^19 elements of K, and 2^26
+    columns times elements."""
+    elems = TK * NKV * D
+    cols = max(56 + elems // (1 << 19), -(-(1 << 26) // elems))
+    return -(-cols // (B * (NQ // NKV)))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,NQ,NKV,D,BLOCK,TK,order", [
+    (1, 28, 4, 128, 1, 10, "scattered"),   # one partial block, very many rows
+    (1, 32, 8, 128, 1, 63, "scattered"),   # one key short of a tile
+    (1, 9, 3, 64, 16, 65, "window"),       # one key over; D = 64
+    (2, 16, 1, 128, 4, 700, "window"),     # batch rows share the staged keys
+    (1, 28, 4, 128, 1, 2100, "window"),    # key splits, a group that does not divide 32
+    (1, 9, 3, 64, 1, 4500, "scattered"),   # more than 64 tiles, any order
+    (1, 32, 8, 128, 16, 1000, "scattered"),
+    (1, 8, 8, 64, 1, 300, "all"),          # no diagonal
+    (1, 28, 4, 128, 8, 200, "none"),       # nothing visible: zeros
+])
+def test_windows_against_fp64(dtype, B, NQ, NKV, D, BLOCK, TK, order):
+    """At the fewest columns that are staged, and one query below (the
+    page-walking kernel)."""
+    most = staged_from(B, NQ, NKV, D, TK)
+    for TQ in (most, most - 1):
+        print(f"[pf-window] {dtype} B={B} NQ={NQ} NKV={NKV} TQ={TQ} D={D} BLOCK={BLOCK} TK={TK} "
+              f"{order}", flush=True)
+        args = inputs(B, NQ, NKV, TQ, D, BLOCK, TK, dtype, seed=TK, order=order)
+        out = ops.position_free_paged_attention(*args, scale=D ** -0.5)
+        if order == "none":
+            torch.cuda.synchronize()
+            assert torch.all(out == 0)
+        else:
+            check(out, reference(*args, D ** -0.5), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_windows_equal_one_query_at_a_time(dtype):
+    """The staged route against the page-walking one, over block sizes, table
+    types, split counts and scales."""
+    TQ = staged_from(1, 28, 4, 128, 500)
+    for BLOCK, tdt, splits, scale in [(1, torch.float32, 0, 0.1), (4, dtype, 1, -0.09),
+                                      (64, torch.float32, 7, 0.0), (1, dtype, 200, 0.2)]:
+        print(f"[pf-window] routes {dtype} BLOCK={BLOCK} tables={tdt} splits={splits} scale={scale}",
+              flush=True)
+        q, kp, vp, table, kpos, qpos, cos, sin = inputs(1, 28, 4, TQ, 128, BLOCK, 500, dtype, seed=5,
+                                                        order="scattered", table_dtype=tdt)
+        out = ops.position_free_paged_attention(q, kp, vp, table, kpos, qpos, cos, sin, scale=scale,
+                                                num_splits=splits)
+        each = torch.cat([ops.position_free_paged_attention(
+            q[:, :, i:i + 1].contiguous(), kp, vp, table, kpos, qpos[i:i + 1], cos, sin, scale=scale)
+            for i in range(TQ)], 2)
+        torch.cuda.synchronize()
+        rel = ((out.double() - each.double()).norm() / each.double().norm()).item()
+        assert rel <= 2 * REL[dtype], (BLOCK, splits, scale, rel)
+
+
+def test_weak_keys_keep_their_weight_in_fp16():
+    """Weights far below fp16's normal range (2^-14 of the largest) still count:
+    one key ahead of 4,000 others whose weights are 2^-16 of its own and whose
+    values all point one way."""
+    print("[pf-window] weak keys", flush=True)
+    TK, D = 4000, 128
+    for TQ in (1, staged_from(1, 2, 1, D, TK)):
+        q = torch.zeros((1, 2, TQ, D), dtype=torch.float16, device="cuda")
+        q[..., D // 2 - 1] = 1.0  # the slowest pair: hardly rotated
+        kp = torch.zeros((TK, 1, 1, D), dtype=torch.float16, device="cuda")
+        kp[0, 0, 0, D // 2 - 1] = 11.09  # 16 ln 2
+        vp = torch.ones((TK, 1, 1, D), dtype=torch.float16, device="cuda")
+        vp[0] = 0
+        table = torch.arange(TK, dtype=torch.int32, device="cuda")
+        qpos = torch.full((TQ,), TK, dtype=torch.int32, device="cuda")
+        cos, sin = ops.rope_cache(TK + 1, D, 1e4, device="cuda")
+        args = (q, kp, vp, table, table, qpos, cos, sin)
+        out = ops.position_free_paged_attention(*args, scale=1.0)
+        check(out, reference(*args, 1.0), torch.float16)

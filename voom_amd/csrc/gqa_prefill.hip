@@ -568,23 +568,21 @@ struct PrefillPlan {
   int row_tiles, splits;
 };
 
-// Row tiles that leave CUs idle are split over keys until there is one workgroup
-// per CU, with at least four 64-key tiles each.  Two per CU are slower (a split's
-// fixed cost: 4 queries over 16,384 tokens, 32/8 heads: 39 against 30 us; 1,024
-// over 1,024: 38 against 28 us); from one per CU on, splitting no longer gains
-// (2,011 over 6,007: 204 against 183 us).  Two tiles per split win at 512 over
-// 512 with 9/3 heads of 64 (13.2 against 14.5 us) and lose at 2 over 4,000 (19.8
-// against 16.4 us).
+// Row tiles that leave CUs idle are split over keys (key_splits), with at least
+// four 64-key tiles each.  Two workgroups per CU from the start are slower (a
+// split's fixed cost: 4 queries over 16,384 tokens, 32/8 heads: 39 against 30 us;
+// 1,024 over 1,024: 38 against 28 us); from one per CU on, splitting no longer
+// gains (2,011 over 6,007: 204 against 183 us).  Two tiles per split win at 512
+// over 512 with 9/3 heads of 64 (13.2 against 14.5 us) and lose at 2 over 4,000
+// (19.8 against 16.4 us).
 PrefillPlan plan_prefill(int B, int NKV, int G, int L, int S) {
   const long long R = static_cast<long long>(L) * G;
   const long long segs = static_cast<long long>(B) * NKV;
-  const int cus = device_cu_count();
   PrefillPlan p;
   p.row_tiles = static_cast<int>((R + NW * kRows - 1) / (NW * kRows));
   const long long wgs = segs * p.row_tiles;
   const int tiles = (S + kKeys - 1) / kKeys;
-  long long s = 1;
-  if (wgs < cus) s = (cus + wgs - 1) / wgs;
+  long long s = key_splits(wgs, device_cu_count());
   if (s > tiles / 4) s = tiles / 4;
   if (s > kMaxSplits) s = kMaxSplits;
   p.splits = s < 1 ? 1 : static_cast<int>(s);

@@ -16,24 +16,26 @@
 //
 // Two attention kernels leave split partials (m, l, o) that pf_reduce_kernel
 // merges:
-//   pf_attention_kernel  bf16 pages, D in {64, 128}: MFMA.  Segments are
+//   pf_attention_kernel  bf16 and fp16 pages, D in {64, 128}: MFMA.  Segments are
 //                        (batch row, kv head); 16 (head, query) columns of a
 //                        segment form the N dimension of one MFMA tile, so each
 //                        key byte is read once for all of them.
-//   pf_generic_kernel    every other element type and head dim (fp32 and fp16
-//                        pages, D any multiple of 32 up to 256): fp32 VALU
-//                        over LDS-staged 32-key blocks, no rounding of P.
+//   pf_generic_kernel    fp32 pages and every other head dim (any multiple of
+//                        32 up to 256): fp32 VALU over LDS-staged 32-key
+//                        blocks, no rounding of P.
 // A segment with more columns than one pass holds (16 for the MFMA kernel,
 // 4096 / D for the generic one) runs as several column passes.  The passes of
 // one piece of work are launched next to each other on the same XCD, so the
 // second pass reads the pages from that XCD's L2.
+// Many columns over 16-bit pages take a route of their own (pf_stage_kernel,
+// pf_window_kernel, below), from where window_pays says.
 //
 // MFMA kernel, per 32-key block a wavefront:
 //   - looks up the 32 page rows and positions (one key per lane),
 //   - loads its K rows as MFMA A operands (16 bytes per lane per k-step),
 //     rotates them in registers -- dims d and d + D/2 sit in k-steps s and
-//     s + D/64 of the same lane -- and rounds them to bf16,
-//   - scores^T[key][column] = K_rot . Q^T with v_mfma_f32_16x16x32_bf16,
+//     s + D/64 of the same lane -- and rounds them to the element type,
+//   - scores^T[key][column] = K_rot . Q^T with v_mfma_f32_16x16x32_{bf16,f16},
 //   - stages the 32 V rows in its own LDS slice and reads V^T operands back
 //     with ds_read_b64_tr_b16, so out^T += V^T . P^T needs no V^T storage.
 // The two 16-key score tiles leave lane (column j, group g) holding keys
@@ -85,6 +87,87 @@ struct EF32 {
   __device__ static void store4(raw* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
 };
 
+// 16-bit element types on the matrix cores.  widen / narrow convert two packed
+// values; weights() packs four softmax weights for P . V in kParts operands and
+// returns their sum: bf16 weights are rounded to bf16 and summed as rounded, fp16
+// weights keep 21 bits in two fp16 halves (hi + lo) and are summed in fp32, so
+// that P stays as good as the fp32 weights of the generic kernel.
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+template <typename E> struct Mma;
+template <> struct Mma<EBf16> {
+  static constexpr int kParts = 1;
+  __device__ __forceinline__ static f32x16 mma32(u32x4 a, u32x4 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+  __device__ __forceinline__ static float weights(float p0, float p1, uint32_t (&w)[kParts],
+                                                  float l) {
+    w[0] = pack_bf16x2(p0, p1);
+    return sum_bf16x2(w[0], l);
+  }
+  __device__ __forceinline__ static f32x4 mma16(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+  __device__ __forceinline__ static f32x2 widen(uint32_t x) {
+    return f32x2{__builtin_bit_cast(float, x << 16), __builtin_bit_cast(float, x & 0xffff0000u)};
+  }
+  __device__ __forceinline__ static uint32_t narrow(float a, float b) { return pack_bf16x2(a, b); }
+  __device__ __forceinline__ static float weights(const float (&p)[4], uint32_t (&w)[kParts][2]) {
+    w[0][0] = pack_bf16x2(p[0], p[1]);
+    w[0][1] = pack_bf16x2(p[2], p[3]);
+    const f32x2 x = widen(w[0][0]), y = widen(w[0][1]);
+    return x[0] + x[1] + y[0] + y[1];
+  }
+};
+template <> struct Mma<EF16> {
+  static constexpr int kParts = 2;
+  // p0, p1 >= 0 as hi + lo: hi rounded toward zero, the exact rest rounded toward
+  // zero again (v_cvt_pkrtz, v_fma_mix: six operations), 2^-21 of p in all.
+  __device__ __forceinline__ static void split(float p0, float p1, uint32_t (&w)[kParts]) {
+    w[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(p0, p1));
+    const f16x2 hi = __builtin_bit_cast(f16x2, w[0]);
+    w[1] = __builtin_bit_cast(
+        uint32_t,
+        __builtin_amdgcn_cvt_pkrtz(__builtin_fmaf(static_cast<float>(hi[0]), -1.f, p0),
+                                   __builtin_fmaf(static_cast<float>(hi[1]), -1.f, p1)));
+  }
+  __device__ __forceinline__ static f32x16 mma32(u32x4 a, u32x4 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+  __device__ __forceinline__ static float weights(float p0, float p1, uint32_t (&w)[kParts],
+                                                  float l) {
+    split(p0, p1, w);
+    return l + (p0 + p1);
+  }
+  __device__ __forceinline__ static f32x4 mma16(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+  __device__ __forceinline__ static f32x2 widen(uint32_t x) {
+    return __builtin_convertvector(__builtin_bit_cast(f16x2, x), f32x2);
+  }
+  __device__ __forceinline__ static uint32_t narrow(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, f16x2));
+  }
+  __device__ __forceinline__ static float weights(const float (&p)[4], uint32_t (&w)[kParts][2]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      uint32_t x[kParts];
+      split(p[2 * i], p[2 * i + 1], x);
+      w[0][i] = x[0];
+      w[1][i] = x[1];
+    }
+    return p[0] + p[1] + p[2] + p[3];
+  }
+};
+
 // Four consecutive table entries as loaded (raw) and as fp32 (cvt): the MFMA
 // kernel keeps the raw chunk in registers while it is in flight and converts
 // it when it is stored to LDS.
@@ -106,6 +189,17 @@ template <> struct TabChunk<EBf16> {
                  __builtin_bit_cast(float, r[0] & 0xffff0000u),
                  __builtin_bit_cast(float, r[1] << 16),
                  __builtin_bit_cast(float, r[1] & 0xffff0000u)};
+  }
+};
+
+template <> struct TabChunk<EF16> {
+  typedef u32x2 raw;
+  __device__ static raw load(const void* base, size_t off) {
+    return *reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(base) + off);
+  }
+  __device__ static f32x4 cvt(raw r) {
+    const f32x2 a = Mma<EF16>::widen(r[0]), b = Mma<EF16>::widen(r[1]);
+    return f32x4{a[0], a[1], b[0], b[1]};
   }
 };
 
@@ -191,9 +285,14 @@ __device__ __forceinline__ long long pf_row_of(int row_lo, int row_hi, int src) 
 // ahead.  Partials are indexed (segment * splits + split, pass * 16 + column).
 // (With 2 or 1 wavefronts per workgroup each thread stages 4-8x the cos/sin
 // chunks of the 8-wavefront shape; those variants get the whole register file.)
-template <int D, int HW, typename TT>
+template <int D, int HW, typename E, typename TT>
 __global__ __launch_bounds__(HW * kWave) __attribute__((amdgpu_waves_per_eu(HW >= 4 ? 2 : 1)))
 void pf_attention_kernel(PfArgs a) {
+  typedef Mma<E> MM;
+  // P of fp16 pages is scaled by 2^kPBias, so that the hi and lo halves of
+  // small weights do not fall into fp16's subnormals (out and l carry the same
+  // factor)
+  constexpr float kPBias = MM::kParts == 2 ? 12.f : 0.f;
   constexpr int KS = D / 32;     // k-steps of the score MFMA
   constexpr int HS = D / 64;     // k-steps in one rotary half
   constexpr int DT = D / 16;     // dim tiles of out^T
@@ -311,13 +410,16 @@ void pf_attention_kernel(PfArgs a) {
 
   // ---- prologue: block blo resident (K in registers; V and cos/sin in
   //      LDS), block blo + 1's table entries loaded ----
-  int rA_lo = 0, rA_hi = 0, kA = 0;   // rows / position of block bi
+  // rows / table position / position for the mask of block bi.  (bf16 pages
+  // mask by the position clamped into the tables, fp16 pages by the given one.)
+  int rA_lo = 0, rA_hi = 0, kA = 0, mA = 0;
   int pgB = 0, psB = 0;               // raw table entry / position of block bi + 1
   u32x4 kc[2][KS];  // K rows of block bi (block bi + 1's once scored)
   if (blo < bhi) {
     int pg, ps;
     pf_key_load(a, blo * kKeys + klane, pg, ps);
     pf_key_finish(a, kvh, blo * kKeys + klane, pg, ps, rA_lo, rA_hi, kA);
+    mA = MM::kParts == 2 ? ps : kA;
     pf_key_load(a, blo + 1 < bhi ? (blo + 1) * kKeys + klane : a.TK, pgB, psB);
     typename TC::raw c0[kCsPerThread];
     u32x4 v0[kVLoads];
@@ -343,6 +445,7 @@ void pf_attention_kernel(PfArgs a) {
     int rB_lo, rB_hi, kB;
     pf_key_finish(a, kvh, more ? (bi + 1) * kKeys + klane : a.TK, pgB, psB, rB_lo, rB_hi,
                   kB);
+    const int mB = MM::kParts == 2 ? psB : kB;
     u32x4 vn[kVLoads];
     typename TC::raw cn[kCsPerThread];
     // cos/sin and V now (they are waited for at the end of this block); K
@@ -353,7 +456,7 @@ void pf_attention_kernel(PfArgs a) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) kp[t][r] = __shfl(kA, 16 * t + 4 * g + r);
+      for (int r = 0; r < 4; ++r) kp[t][r] = __shfl(mA, 16 * t + 4 * g + r);
     }
     __builtin_amdgcn_sched_barrier(0);
 
@@ -374,21 +477,19 @@ void pf_attention_kernel(PfArgs a) {
         u32x4 lo_out, hi_out;
 #pragma unroll
         for (int wv = 0; wv < 4; ++wv) {
-          const uint32_t xa = kc[t][s][wv];
-          const uint32_t xb = kc[t][s + HS][wv];
+          const f32x2 av = MM::widen(kc[t][s][wv]);
+          const f32x2 bv = MM::widen(kc[t][s + HS][wv]);
           float ra[2], rb[2];
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
-            const float av = __builtin_bit_cast(float, h ? (xa & 0xffff0000u) : (xa << 16));
-            const float bv = __builtin_bit_cast(float, h ? (xb & 0xffff0000u) : (xb << 16));
             const int e = 2 * wv + h;
             const float c = e < 4 ? cA[e] : cB[e - 4];
             const float sv = e < 4 ? sA[e] : sB[e - 4];
-            ra[h] = av * c - bv * sv;
-            rb[h] = bv * c + av * sv;
+            ra[h] = av[h] * c - bv[h] * sv;
+            rb[h] = bv[h] * c + av[h] * sv;
           }
-          lo_out[wv] = pack_bf16x2(ra[0], ra[1]);
-          hi_out[wv] = pack_bf16x2(rb[0], rb[1]);
+          lo_out[wv] = MM::narrow(ra[0], ra[1]);
+          hi_out[wv] = MM::narrow(rb[0], rb[1]);
         }
         kc[t][s] = lo_out;
         kc[t][s + HS] = hi_out;
@@ -396,9 +497,7 @@ void pf_attention_kernel(PfArgs a) {
       f32x4 acc_s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
-        acc_s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kc[t][s]),
-                                                        __builtin_bit_cast(bf16x8, qop[s]),
-                                                        acc_s, 0, 0, 0);
+        acc_s = MM::mma16(kc[t][s], qop[s], acc_s);
       }
       sc[t] = acc_s;
     }
@@ -422,37 +521,42 @@ void pf_attention_kernel(PfArgs a) {
     const float m_new = fmaxf(m_run, mb);
     const float alpha = m_new == m_run ? 1.f : fast_exp2(m_run - m_new);
     m_run = m_new;
-    u32x4 pk;
+    u32x4 pk[MM::kParts];
     float ps = 0.f;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       float p[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) p[r] = x[t][r] == -INFINITY ? 0.f : fast_exp2(x[t][r] - m_new);
-      const uint32_t w0 = pack_bf16x2(p[0], p[1]);
-      const uint32_t w1 = pack_bf16x2(p[2], p[3]);
-      pk[2 * t] = w0;
-      pk[2 * t + 1] = w1;
-      ps += __builtin_bit_cast(float, w0 << 16) + __builtin_bit_cast(float, w0 & 0xffff0000u) +
-            __builtin_bit_cast(float, w1 << 16) + __builtin_bit_cast(float, w1 & 0xffff0000u);
+      for (int r = 0; r < 4; ++r)
+        p[r] = x[t][r] == -INFINITY ? 0.f : fast_exp2(x[t][r] - m_new + kPBias);
+      uint32_t pw[MM::kParts][2];
+      ps += MM::weights(p, pw);
+#pragma unroll
+      for (int part = 0; part < MM::kParts; ++part) {
+        pk[part][2 * t] = pw[part][0];
+        pk[part][2 * t + 1] = pw[part][1];
+      }
     }
     l_lane = l_lane * alpha + ps;
 
     // ---- out^T[dims][columns] += V^T . P^T ----
 #pragma unroll
     for (int d = 0; d < DT; ++d) acc[d] *= alpha;
-    const bf16x8 pb = __builtin_bit_cast(bf16x8, pk);
     // lane i16 of group g addresses key row 4g + i16/4 (and +16) at dims
     // 16dt + 4*(i16%4): after the transpose lane l holds keys 4g..4g+3 (and
     // 16 + 4g..) of dim 16dt + l%16
     const uint16_t* vb = vs + (4 * g + (i16 >> 2)) * kVRow + 4 * (i16 & 3);
-#pragma unroll
-    for (int d = 0; d < DT; ++d) {
+    auto read_v = [&](int d) {
       const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(vb + 16 * d));
       const bf16x4 hi =
           __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(vb + 16 * kVRow + 16 * d));
-      const bf16x8 av = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-      acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, pb, acc[d], 0, 0, 0);
+      return __builtin_bit_cast(u32x4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      const u32x4 av = read_v(d);
+#pragma unroll
+      for (int part = 0; part < MM::kParts; ++part) acc[d] = MM::mma16(av, pk[part], acc[d]);
     }
 
     // ---- block bi + 1's V rows into the slice once this block's reads of
@@ -467,6 +571,7 @@ void pf_attention_kernel(PfArgs a) {
     rA_lo = rB_lo;
     rA_hi = rB_hi;
     kA = kB;
+    mA = mB;
     pgB = pgC;
     psB = psC;
   }
@@ -808,13 +913,572 @@ __global__ __launch_bounds__(kRedWaves * kWave) void pf_reduce_kernel(PfArgs a,
             res * inv);
 }
 
-template <int D, typename TT>
+// ---- windows: many columns over 16-bit pages ----------------------------------
+// A segment with many (query, head) columns is bound by matrix work, and the
+// passes of pf_attention_kernel rotate every key again for each 16 columns.  So
+// pf_stage_kernel first gathers the pages once, rotates the keys, and leaves
+// contiguous 32-key blocks in the workspace, K [32][D] and V^T [D][32], with the
+// positions for the mask; pf_window_kernel then runs 64-key tiles of them against
+// 32 rows per wavefront, as gqa_prefill_kernel does over pages of rotated keys:
+// the rows of a kv head are its (batch row, query, head of the group) columns,
+// scores^T and out^T on 32x32x16 MFMAs, P^T in registers, the scores one tile
+// ahead of P . V, operands straight into LDS, one barrier per tile.  250 queries
+// over 8,003 keys (28q/4kv, D = 128): fp16 3,866 us in the generic kernel, 446 in
+// pf_attention_kernel's 110 passes, 78 here (11 staging, 60 the window kernel, 5
+// the merge of its splits); bf16 449 and 65 us.
+constexpr int kWinWaves = 4;
+constexpr int kWinRows = 32;                       // rows of a wavefront
+constexpr int kWinTile = kWinWaves * kWinRows;     // rows of a workgroup
+constexpr int kWinKeys = 64;                       // keys of a tile
+constexpr int kWinAhead = 4;                       // operand reads ahead of the MFMAs
+constexpr int kWinMaxSplits = 64;
+
+struct WinArgs {
+  PfArgs p;
+  uint16_t* k_blk;      // [NKV, nblk, 32, D]
+  uint16_t* v_blk;      // [NKV, nblk, D, 32]
+  int32_t* pos;         // [nblk * 32] positions for the mask (INT_MAX past the last key)
+  int2* span;           // [nblk] smallest and largest of them
+  int nblk;             // 32-key blocks, even
+  int R;                // rows of a kv head: B * TQ * G, the head fastest
+  int row_tiles, splits;
+  int work, per_xcd, xcd_cus;
+  float scale;          // |softmax scale| in log2 units, > 0; its sign is applied to q
+  uint32_t q_keep, q_flip;
+};
+
+// Workgroup (blk, kvh): one 32-key block.
+template <int D, typename E, typename TT>
+__global__ __launch_bounds__(256) void pf_stage_kernel(WinArgs w) {
+  typedef Mma<E> MM;
+  typedef TabChunk<TT> TC;
+  constexpr int kPairs = kKeys * D / 16;   // (8 dims, their rotary partners) of a key
+  constexpr int kChunks = kKeys * D / 8;   // 16-byte chunks of V
+  constexpr int kVs = D + 8;
+  __shared__ long long row[kKeys];
+  __shared__ int at[kKeys];
+  __shared__ __attribute__((aligned(16))) uint16_t vs[kKeys * kVs];
+  const PfArgs& a = w.p;
+  const int t = threadIdx.x;
+  const int blk = blockIdx.x / a.NKV;
+  const int kvh = blockIdx.x - blk * a.NKV;
+  if (t < kKeys) {
+    const int key = blk * kKeys + t;
+    long long r = -1;
+    int p = 0, m = INT_MAX;
+    if (key < a.TK) {
+      const int tb = key / a.BLOCK;
+      int page = a.table[tb];
+      page = static_cast<unsigned>(page) < static_cast<unsigned>(a.P) ? page : 0;
+      r = (static_cast<long long>(page) * a.NKV + kvh) * a.BLOCK + (key - tb * a.BLOCK);
+      const int raw = a.k_pos[key];
+      p = raw < 0 ? 0 : (raw >= a.max_pos ? a.max_pos - 1 : raw);
+      m = MM::kParts == 2 ? raw : p;  // as pf_attention_kernel masks
+    }
+    row[t] = r;
+    at[t] = p;
+    if (kvh == 0) {
+      w.pos[blk * kKeys + t] = m;
+      int lo = m, hi = m;
+#pragma unroll
+      for (int o = kKeys / 2; o > 0; o >>= 1) {
+        lo = min(lo, __shfl_xor(lo, o, kKeys));
+        hi = max(hi, __shfl_xor(hi, o, kKeys));
+      }
+      if (t == 0) w.span[blk] = make_int2(lo, hi);
+    }
+  }
+  __syncthreads();
+  const uint16_t* kp = static_cast<const uint16_t*>(a.k_pages);
+  const uint16_t* vp = static_cast<const uint16_t*>(a.v_pages);
+  const size_t out = (static_cast<size_t>(kvh) * w.nblk + blk) * (kKeys * D);
+  for (int i = t; i < kChunks; i += 256) {
+    const int key = i / (D / 8), c = i % (D / 8);
+    const u32x4 z = {0u, 0u, 0u, 0u};
+    const u32x4 v = row[key] < 0 ? z : __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
+                                           vp + row[key] * D + 8 * c));
+    *reinterpret_cast<u32x4*>(vs + key * kVs + 8 * c) = v;
+  }
+  for (int i = t; i < kPairs; i += 256) {
+    const int key = i / (D / 16), c = i % (D / 16);
+    const uint16_t* kr = kp + (row[key] < 0 ? 0 : row[key]) * D + 8 * c;
+    const u32x4 x = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kr));
+    const u32x4 y = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kr + D / 2));
+    const size_t to = static_cast<size_t>(at[key]) * (D / 2) + 8 * c;
+    const f32x4 c0 = TC::cvt(TC::load(a.cos_t, to)), c1 = TC::cvt(TC::load(a.cos_t, to + 4));
+    const f32x4 s0 = TC::cvt(TC::load(a.sin_t, to)), s1 = TC::cvt(TC::load(a.sin_t, to + 4));
+    u32x4 lo, hi;
+#pragma unroll
+    for (int wv = 0; wv < 4; ++wv) {
+      const f32x2 av = MM::widen(x[wv]), bv = MM::widen(y[wv]);
+      float ra[2], rb[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int e = 2 * wv + h;
+        const float cv = e < 4 ? c0[e] : c1[e - 4];
+        const float sv = e < 4 ? s0[e] : s1[e - 4];
+        ra[h] = av[h] * cv - bv[h] * sv;
+        rb[h] = bv[h] * cv + av[h] * sv;
+      }
+      lo[wv] = MM::narrow(ra[0], ra[1]);
+      hi[wv] = MM::narrow(rb[0], rb[1]);
+    }
+    if (row[key] < 0) lo = hi = u32x4{0u, 0u, 0u, 0u};
+    uint16_t* o = w.k_blk + out + key * D + 8 * c;
+    *reinterpret_cast<u32x4*>(o) = lo;
+    *reinterpret_cast<u32x4*>(o + D / 2) = hi;
+  }
+  __syncthreads();
+  for (int i = t; i < kChunks; i += 256) {
+    const int d = i >> 2, c = i & 3;
+    u32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      v[e] = vs[(8 * c + 2 * e) * kVs + d] |
+             (static_cast<uint32_t>(vs[(8 * c + 2 * e + 1) * kVs + d]) << 16);
+    *reinterpret_cast<u32x4*>(w.v_blk + out + d * kKeys + 8 * c) = v;
+  }
+}
+
+// Key (0..31 of a block) that row r of the score tile holds: lane half h then
+// has keys 8h..8h+7 in its first eight accumulators and 16+8h.. in the others,
+// which is the order its P^T operand needs.
+__device__ __forceinline__ int win_key_of_row(int r) {
+  return 16 * (r >> 4) + 8 * ((r >> 2) & 1) + 4 * ((r >> 3) & 1) + (r & 3);
+}
+// Chunk c (16 bytes) of K row r sits at c ^ win_k_swizzle(r) in LDS.
+template <int D>
+__device__ __forceinline__ int win_k_swizzle(int r) {
+  return D == 128 ? (r & 15) : ((r >> 1) & 7);
+}
+
+template <int D, typename E>
+__global__ __launch_bounds__(kWinWaves * kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void pf_window_kernel(WinArgs wa, uint16_t* out) {
+  typedef Mma<E> MM;
+  typedef __attribute__((address_space(3))) void lds_void;
+  constexpr int NW = kWinWaves;
+  constexpr int kBlkElems = kKeys * D;
+  constexpr int kPieces = kBlkElems / 512;  // 1 KiB loads per block
+  constexpr int kLoads = 4 * kPieces / NW;  // per wavefront and stage
+  constexpr int kCpr = D / 8;               // 16-byte chunks of a K row
+  constexpr int KS = D / 16;
+  constexpr int DT = D / 32;
+  constexpr int kA = kWinAhead;
+  // P of fp16 pages is scaled by 2^kPBias (see pf_attention_kernel)
+  constexpr float kPBias = MM::kParts == 2 ? 12.f : 0.f;
+  // masks of __builtin_amdgcn_sched_group_barrier
+  constexpr int kValu = 0x002, kMfma = 0x008, kVmemRead = 0x020, kDsRead = 0x100, kTrans = 0x400;
+  static_assert(kPieces >= NW && (kLoads == 8 || kLoads == 4), "loads of a stage");
+  // K block 0, K block 1, V^T block 0, V^T block 1; two distinct objects, so that
+  // reads of one provably miss the other's pending direct-to-LDS loads
+  __shared__ __attribute__((aligned(1024))) uint16_t tile_a[4 * kBlkElems];
+  __shared__ __attribute__((aligned(1024))) uint16_t tile_b[4 * kBlkElems];
+  const PfArgs& a = wa.p;
+
+  // as in gqa_prefill_kernel: consecutive work items of one XCD share a kv head
+  const int bid = static_cast<int>(blockIdx.x);
+  int slot = bid >> 3;
+  if (slot >= wa.xcd_cus && wa.per_xcd <= 2 * wa.xcd_cus)
+    slot = wa.per_xcd - 1 - (slot - wa.xcd_cus);
+  const int wk = (bid & 7) * wa.per_xcd + slot;
+  if (wk >= wa.work) return;
+  const int per_seg = wa.row_tiles * wa.splits;
+  const int kvh = wk / per_seg;
+  const int in_seg = wk - kvh * per_seg;
+  const int rt = wa.row_tiles - 1 - in_seg / wa.splits;
+  const int split = in_seg % wa.splits;
+
+  const int lane = threadIdx.x & (kWave - 1);
+  const int w = uniform(threadIdx.x / kWave) & (NW - 1);
+  const int l32 = lane & 31;
+  const int lh = lane >> 5;
+
+  // this lane's row: (batch row, query, head)
+  const int row = rt * kWinTile + w * kWinRows + l32;
+  const bool row_ok = row < wa.R;
+  const int rc = row_ok ? row : wa.R - 1;
+  const int bt = rc / a.G;
+  const int b = bt / a.TQ;
+  const int tq = bt - b * a.TQ;
+  const size_t qrow =
+      (static_cast<size_t>(b) * a.NQ + kvh * a.G + (rc - bt * a.G)) * a.TQ + tq;
+  const int qpos = a.q_pos[tq];
+  int q_lo = qpos, q_hi = qpos;  // of the wavefront's rows
+#pragma unroll
+  for (int o = 16; o > 0; o >>= 1) {
+    q_lo = min(q_lo, __shfl_xor(q_lo, o));
+    q_hi = max(q_hi, __shfl_xor(q_hi, o));
+  }
+  // keys end (for this workgroup) with the last block that one of its rows sees
+  int n_tiles;
+  {
+    int top = INT_MIN;
+#pragma unroll
+    for (int i = 0; i < kWinTile / kWave; ++i) {
+      const int r = min(rt * kWinTile + i * kWave + lane, wa.R - 1);
+      top = max(top, a.q_pos[(r / a.G) % a.TQ]);
+    }
+    int last = -1;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) top = max(top, __shfl_xor(top, o));
+    for (int i = lane; i < wa.nblk; i += kWave) {
+      if (i * kKeys < a.TK && wa.span[i].x <= top) last = i;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) last = max(last, __shfl_xor(last, o));
+    n_tiles = uniform(last + 2) >> 1;
+  }
+  const int t_lo = static_cast<int>(static_cast<long long>(split) * n_tiles / wa.splits);
+  const int t_hi = static_cast<int>(static_cast<long long>(split + 1) * n_tiles / wa.splits);
+
+  u32x4 qop[KS];
+  auto load_q = [&]() {
+    const uint16_t* qh = static_cast<const uint16_t*>(a.q) + qrow * D + 8 * lh;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      qop[s] = *reinterpret_cast<const u32x4*>(qh + 16 * s);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) qop[s][i] = (qop[s][i] & wa.q_keep) ^ wa.q_flip;
+    }
+  };
+
+  // Per tile of win .. win + 63, one bit each: every row of the wavefront sees
+  // all its keys; some row sees one.
+  int win = 0;
+  unsigned long long whole_bits = 0, seen_bits = 0;
+  auto look_ahead = [&](int t) {
+    win = t;
+    const int mine = t + lane;
+    int2 s0 = make_int2(INT_MAX, INT_MAX), s1 = s0;
+    if (2 * mine < wa.nblk) {
+      s0 = wa.span[2 * mine];
+      s1 = wa.span[2 * mine + 1];
+    }
+    whole_bits = __builtin_amdgcn_ballot_w64((mine + 1) * kWinKeys <= a.TK && s0.y <= q_lo &&
+                                             s1.y <= q_lo);
+    seen_bits = __builtin_amdgcn_ballot_w64(mine * kWinKeys < a.TK && (s0.x <= q_hi || s1.x <= q_hi));
+    wait_vmem_all();
+  };
+  auto whole = [&](int t) { return ((whole_bits >> (t - win)) & 1) != 0; };
+  auto seen = [&](int t) { return ((seen_bits >> (t - win)) & 1) != 0; };
+
+  // Stage t holds K of tile t + 1 and V^T of tile t.
+  const uint16_t* kseg = wa.k_blk + static_cast<size_t>(kvh) * wa.nblk * kBlkElems;
+  const uint16_t* vseg = wa.v_blk + static_cast<size_t>(kvh) * wa.nblk * kBlkElems;
+  auto load_piece = [&](int i, int t, uint16_t* dst) {
+    const int p = w + NW * i;
+    const int j = (p / kPieces) & 1;
+    const int sub = p % kPieces;
+    const bool is_v = i >= kLoads / 2;
+    const uint16_t* base =
+        (is_v ? vseg + static_cast<size_t>(max(t, 0)) * (2 * kBlkElems)
+              : kseg + static_cast<size_t>(min(t + 1, t_hi - 1)) * (2 * kBlkElems)) +
+        j * kBlkElems;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(base), static_cast<short>(0), kBlkElems * 2, 0x00020000);
+    const int krow = sub * (kWave / kCpr) + lane / kCpr;
+    const int ksrc = krow * (D * 2) + 16 * ((lane % kCpr) ^ win_k_swizzle<D>(krow));
+    const int vrow = sub * 16 + (lane >> 2);
+    const int vsrc = vrow * (kKeys * 2) + 16 * ((lane & 3) ^ ((lane >> 4) & 3));
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)(dst + p * 512), 16, is_v ? vsrc : ksrc,
+                                             0, 0, 0);
+  };
+  auto load_stage = [&](int t, uint16_t* dst) {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) load_piece(i, t, dst);
+  };
+
+  const int key = win_key_of_row(l32);
+  const int k_lane = key * (D * 2) + 16 * (lh ^ win_k_swizzle<D>(key));
+  int v_lane[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+    v_lane[ks] = l32 * (kKeys * 2) + 16 * ((2 * ks + lh) ^ ((l32 >> 2) & 3));
+
+  f32x16 acc[DT];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) acc[d] = f32x16{};
+  float m = -INFINITY;
+  float l = 0.f;
+
+  typedef f32x16 Scores[2];  // accumulator i of block j: key 32 j + 16 (i / 8) + 8 lh + i % 8
+  auto mask_scores = [&](int t, Scores& sc) {
+    const int32_t* kp = wa.pos + t * kWinKeys + 8 * lh;
+#pragma unroll
+    for (int jk = 0; jk < 4; ++jk) {
+      const int4 p0 = *reinterpret_cast<const int4*>(kp + 16 * jk);
+      const int4 p1 = *reinterpret_cast<const int4*>(kp + 16 * jk + 4);
+      const int ps[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+      const int lim = a.TK - t * kWinKeys - 16 * jk - 8 * lh;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float x = sc[jk >> 1][8 * (jk & 1) + i];
+        sc[jk >> 1][8 * (jk & 1) + i] = i < lim && ps[i] <= qpos ? x : -INFINITY;
+      }
+    }
+  };
+  auto max_of = [&](const Scores& sc) {
+    float mx = fmaxf(sc[0][0], sc[1][0]);
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mx = fmaxf(fmaxf(mx, sc[0][i]), sc[1][i]);
+    return mx;
+  };
+  auto raise = [&](float mx) {
+    mx = fmaxf(mx, __shfl_xor(mx, 32)) * wa.scale;
+    if (__builtin_amdgcn_ballot_w64(mx > m) == 0) return;
+    const float mn = fmaxf(m, mx);
+    float alpha = mn == -INFINITY ? 1.f : fast_exp2(m - mn);
+    asm volatile("" : "+v"(alpha));  // keeps the rescaling inside the branch
+    m = mn;
+    l *= alpha;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) acc[d] *= alpha;
+  };
+  auto read_k = [&](const uint16_t* tile, int i) {  // i = 2 s + j
+    return *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(tile) +
+                                           (i & 1) * (kBlkElems * 2) + (k_lane ^ (32 * (i >> 1))));
+  };
+  auto read_v = [&](const uint16_t* tile, int i) {  // i = (2 j + ks) * DT + d
+    const int j = i / (2 * DT), ks = (i / DT) & 1, d = i % DT;
+    return *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(tile) +
+                                           (2 + j) * (kBlkElems * 2) + d * (32 * kKeys * 2) +
+                                           v_lane[ks]);
+  };
+  auto first_scores = [&](const uint16_t* tile, Scores& sc) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) sc[j] = f32x16{};
+#pragma unroll
+    for (int i = 0; i < 2 * KS; ++i) sc[i & 1] = MM::mma32(read_k(tile, i), qop[i >> 1], sc[i & 1]);
+  };
+  typedef u32x4 Weights[MM::kParts][4];  // P^T operands of the four 16-key steps
+  auto form_p = [&](int e, const Scores& sc, float mref, Weights& pk) {
+    const int j = e >> 3, n = 2 * (e & 7);
+    uint32_t pw[MM::kParts];
+    l = MM::weights(fast_exp2(__builtin_fmaf(sc[j][n], wa.scale, kPBias - mref)),
+                    fast_exp2(__builtin_fmaf(sc[j][n + 1], wa.scale, kPBias - mref)), pw, l);
+#pragma unroll
+    for (int part = 0; part < MM::kParts; ++part)
+      pk[part][2 * j + (n >> 3)][(n & 7) >> 1] = pw[part];
+  };
+
+  // Tile t where every row of the wavefront sees all of tiles t and t + 1.
+  auto whole_tile = [&](int t, const uint16_t* tile, uint16_t* next, const Scores& sc,
+                        Scores& nx) {
+    const float mref = m;
+    Weights pk;
+    u32x4 ring[kA];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) nx[j] = f32x16{};
+#pragma unroll
+    for (int i = 0; i < kA; ++i) ring[i] = read_k(tile, i);
+    __builtin_amdgcn_sched_group_barrier(kDsRead, kA, 0);
+#pragma unroll
+    for (int i = 0; i < 2 * KS; ++i) {
+      nx[i & 1] = MM::mma32(ring[i % kA], qop[i >> 1], nx[i & 1]);
+      __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+      if (i + kA < 2 * KS) {
+        ring[i % kA] = read_k(tile, i + kA);
+        __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
+      }
+      if (i * kLoads / (2 * KS) != (i + 1) * kLoads / (2 * KS)) {
+        load_piece(i * kLoads / (2 * KS), t + 1, next);
+        __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
+      }
+#pragma unroll
+      for (int e = i * 16 / (2 * KS); e < (i + 1) * 16 / (2 * KS); ++e) {
+        form_p(e, sc, mref, pk);
+        __builtin_amdgcn_sched_group_barrier(kValu, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(kTrans, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(kValu, MM::kParts == 2 ? 8 : 2, 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < kA; ++i) ring[i] = read_v(tile, i);
+    __builtin_amdgcn_sched_group_barrier(kDsRead, kA, 1);
+    float mx = fmaxf(nx[0][0], nx[1][0]);
+#pragma unroll
+    for (int i = 0; i < 4 * DT; ++i) {
+#pragma unroll
+      for (int part = 0; part < MM::kParts; ++part)
+        acc[i % DT] = MM::mma32(ring[i % kA], pk[part][i / DT], acc[i % DT]);
+      __builtin_amdgcn_sched_group_barrier(kMfma, MM::kParts, 1);
+      if (i + kA < 4 * DT) {
+        ring[i % kA] = read_v(tile, i + kA);
+        __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 1);
+      }
+#pragma unroll
+      for (int e = i * 16 / (4 * DT); e < (i + 1) * 16 / (4 * DT); ++e) {
+        if (e == 0) continue;
+        mx = fmaxf(fmaxf(mx, nx[0][e]), nx[1][e]);
+        __builtin_amdgcn_sched_group_barrier(kValu, 1, 1);
+      }
+    }
+    raise(mx);
+  };
+
+  // Any tile t: its scores are in sc, which then takes those of tile t + 1.
+  auto edge_tile = [&](int t, const uint16_t* tile, Scores& sc) {
+    if (seen(t)) {
+      const float mref = m == -INFINITY ? 0.f : m;  // nothing visible yet: P = 0
+      Weights pk;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) form_p(e, sc, mref, pk);
+#pragma unroll
+      for (int i = 0; i < 4 * DT; ++i) {
+        const u32x4 vv = read_v(tile, i);
+#pragma unroll
+        for (int part = 0; part < MM::kParts; ++part)
+          acc[i % DT] = MM::mma32(vv, pk[part][i / DT], acc[i % DT]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (t + 1 < t_hi && seen(t + 1)) {
+      first_scores(tile, sc);
+      mask_scores(t + 1, sc);
+      raise(max_of(sc));
+    }
+  };
+
+  Scores sc_a, sc_b;
+  auto landed = [&]() {
+    wait_vmem_all();
+    lds_barrier();
+  };
+  if (t_lo < t_hi) {
+    look_ahead(t_lo);
+#pragma unroll
+    for (int i = 0; i < kLoads / 2; ++i) load_piece(i, t_lo - 1, tile_b);
+    load_q();
+    load_stage(t_lo, tile_a);
+    // the first tile's K has landed (gfx9 encoding: vmcnt kLoads, lgkmcnt 15)
+    if constexpr (kLoads == 8) __builtin_amdgcn_s_waitcnt(0x0F78);
+    else __builtin_amdgcn_s_waitcnt(0x0F74);
+    lds_barrier();
+    if (seen(t_lo)) {
+      first_scores(tile_b, sc_a);
+      mask_scores(t_lo, sc_a);
+      raise(max_of(sc_a));
+    }
+  }
+  for (int t = t_lo; t < t_hi;) {
+    // pairs of tiles that are whole, the one after them (whose scores run
+    // ahead) too; otherwise a pair of any kind
+    while (t + 2 < t_hi && t - win < 60 && ((whole_bits >> (t - win)) & 7) == 7) {
+      landed();
+      whole_tile(t, tile_a, tile_b, sc_a, sc_b);
+      landed();
+      whole_tile(t + 1, tile_b, tile_a, sc_b, sc_a);
+      t += 2;
+    }
+    landed();
+    if (t - win >= 60) look_ahead(t);
+    if (t + 1 < t_hi) load_stage(t + 1, tile_b);
+    edge_tile(t, tile_a, sc_a);
+    if (t + 1 >= t_hi) break;
+    landed();
+    if (t + 2 < t_hi) load_stage(t + 2, tile_a);
+    edge_tile(t + 1, tile_b, sc_a);
+    t += 2;
+  }
+
+  const float lt = l + __shfl_xor(l, 32);
+  if (!row_ok) return;
+  if (wa.splits == 1) {
+    const float inv = lt > 0.f ? 1.f / lt : 0.f;
+    uint16_t* o = out + qrow * D + 4 * lh;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        E::store4(o + 32 * d + 8 * i, f32x4{acc[d][4 * i], acc[d][4 * i + 1], acc[d][4 * i + 2],
+                                            acc[d][4 * i + 3]} * inv);
+    }
+    return;
+  }
+  const size_t p = (static_cast<size_t>(kvh) * wa.R + row) * wa.splits + split;
+  float* o = a.part_o + p * D + 4 * lh;
+#pragma unroll
+  for (int d = 0; d < DT; ++d) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<f32x4*>(o + 32 * d + 8 * i) =
+          f32x4{acc[d][4 * i], acc[d][4 * i + 1], acc[d][4 * i + 2], acc[d][4 * i + 3]};
+  }
+  if (lh == 0) {
+    a.part_ml[p * 2 + 0] = m;
+    a.part_ml[p * 2 + 1] = lt;
+  }
+}
+
+// One wavefront per row: merges its key splits (at most 64) into the output.
+template <int D, typename E>
+__global__ __launch_bounds__(256) void pf_window_combine_kernel(WinArgs wa, uint16_t* out,
+                                                                int rows) {
+  constexpr int kLanes = D / 4;           // lanes across a row, four dims each
+  constexpr int kSide = kWave / kLanes;   // splits side by side
+  const PfArgs& a = wa.p;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int task = blockIdx.x * 4 + uniform(threadIdx.x / kWave);
+  if (task >= rows) return;
+  const int kvh = task / wa.R;
+  const int row = task - kvh * wa.R;
+  const int bt = row / a.G;
+  const int b = bt / a.TQ;
+  const size_t p0 = static_cast<size_t>(task) * wa.splits;
+  const bool live = lane < wa.splits;
+  const float2 ml = reinterpret_cast<const float2*>(a.part_ml)[p0 + (live ? lane : 0)];
+  const float M = wave_max_uniform(live ? ml.x : -INFINITY);
+  // a split that holds no visible key of the row left m = -inf, l = 0
+  const float wt = live && ml.x != -INFINITY ? fast_exp2(ml.x - M) : 0.f;
+  const float lt = wave_sum_uniform(live ? ml.y * wt : 0.f);
+  const int c = lane % kLanes, side = lane / kLanes;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < wa.splits; s0 += 4 * kSide) {
+    f32x4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int s = min(s0 + u * kSide + side, wa.splits - 1);
+      v[u] = *reinterpret_cast<const f32x4*>(a.part_o + (p0 + s) * D + 4 * c);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int s = s0 + u * kSide + side;
+      const float ws = __shfl(wt, s & (kWave - 1));
+      if (s < wa.splits) acc += v[u] * ws;
+    }
+  }
+#pragma unroll
+  for (int x = kLanes; x < kWave; x <<= 1) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] += __shfl_xor(acc[e], x);
+  }
+  if (side != 0) return;
+  const float inv = lt > 0.f ? 1.f / lt : 0.f;
+  const size_t qrow =
+      (static_cast<size_t>(b) * a.NQ + kvh * a.G + (row - bt * a.G)) * a.TQ + (bt - b * a.TQ);
+  E::store4(out + qrow * D + 4 * c, acc * inv);
+}
+
+template <int D, typename E, typename TT>
 void launch_pf_attention(int hw, dim3 grid, dim3 block, hipStream_t stream, const PfArgs& a) {
   switch (hw) {
-    case 8: hipLaunchKernelGGL((pf_attention_kernel<D, 8, TT>), grid, block, 0, stream, a); break;
-    case 4: hipLaunchKernelGGL((pf_attention_kernel<D, 4, TT>), grid, block, 0, stream, a); break;
-    case 2: hipLaunchKernelGGL((pf_attention_kernel<D, 2, TT>), grid, block, 0, stream, a); break;
-    default: hipLaunchKernelGGL((pf_attention_kernel<D, 1, TT>), grid, block, 0, stream, a); break;
+    case 8: hipLaunchKernelGGL((pf_attention_kernel<D, 8, E, TT>), grid, block, 0, stream, a); break;
+    case 4: hipLaunchKernelGGL((pf_attention_kernel<D, 4, E, TT>), grid, block, 0, stream, a); break;
+    case 2: hipLaunchKernelGGL((pf_attention_kernel<D, 2, E, TT>), grid, block, 0, stream, a); break;
+    default: hipLaunchKernelGGL((pf_attention_kernel<D, 1, E, TT>), grid, block, 0, stream, a); break;
+  }
+}
+template <typename E>
+void launch_pf_attention_e(int D, bool f32_tab, int hw, dim3 grid, dim3 block, hipStream_t stream,
+                           const PfArgs& a) {
+  if (D == 128) {
+    if (f32_tab) launch_pf_attention<128, E, EF32>(hw, grid, block, stream, a);
+    else launch_pf_attention<128, E, E>(hw, grid, block, stream, a);
+  } else {
+    if (f32_tab) launch_pf_attention<64, E, EF32>(hw, grid, block, stream, a);
+    else launch_pf_attention<64, E, E>(hw, grid, block, stream, a);
   }
 }
 
@@ -825,18 +1489,57 @@ struct PfPlan {
   bool mfma;
   int hw;      // kv heads per workgroup (MFMA kernel)
   int ncg, passes, ncp, splits;
-  size_t o_bytes, ws_bytes;
+  bool window;            // the window kernels
+  int row_tiles, nblk;
+  size_t o_bytes;         // the partial outputs' bytes (the statistics follow)
+  size_t stage_at, pos_at, span_at;  // window: the staged blocks in the workspace
+  size_t ws_bytes;
 };
 
+// Columns times keys from which staging the pages pays: the staged route costs a
+// pass over the pages (10 us at 4 MiB of K, 80 us at 64 MiB) and about 19 us of
+// launches and fill, the page-walking one a rotation of every key per 16 columns.
+// Measured (bf16, walking / staged, us): 28q/4kv, D = 128, 8,003 keys: 56 columns
+// 29.5 / 34.4, 112 columns 45 / 35, 1,750 columns 449 / 76; 32q/8kv, 32,768 keys:
+// 64 columns 89 / 100; 2,000 keys: 32 columns 22.5 / 22.4, 64 columns 28.8 / 23.9;
+// 9q/3kv, D = 64, 20,000 keys: 72 columns 34.4 / 34.1, 144 columns 49 / 40; 500
+// keys: 300 columns 16 / 20.
+bool window_pays(long long cols, int TK, int NKV, int D) {
+  const long long elems = static_cast<long long>(TK) * NKV * D;
+  return cols >= 56 + elems / (1 << 19) && cols * elems >= 1LL << 26;
+}
+
+size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
+
 PfPlan pf_plan(int B, int NQ, int TQ, int NKV, int D, int TK, int dtype, int num_splits) {
-  PfPlan p;
+  PfPlan p = {};
   const int NC = NQ / NKV * TQ;
-  p.mfma = dtype == VOOM_DTYPE_BF16 && (D == 64 || D == 128);
+  const int nb = (TK + kKeys - 1) / kKeys;
+  p.mfma = dtype != VOOM_DTYPE_F32 && (D == 64 || D == 128);
+  p.window = p.mfma && window_pays(static_cast<long long>(B) * NC, TK, NKV, D);
+  if (p.window) {
+    const long long R = static_cast<long long>(B) * NC;
+    p.row_tiles = static_cast<int>((R + kWinTile - 1) / kWinTile);
+    p.nblk = (nb + 1) & ~1;
+    long long s = num_splits > 0 ? num_splits
+                                 : key_splits(static_cast<long long>(NKV) * p.row_tiles,
+                                              device_cu_count());
+    if (num_splits <= 0 && s > p.nblk / 8) s = p.nblk / 8;  // four 64-key tiles each
+    if (s > kWinMaxSplits) s = kWinMaxSplits;
+    p.splits = s < 1 ? 1 : static_cast<int>(s);
+    const size_t rows = p.splits > 1 ? static_cast<size_t>(NKV) * R * p.splits : 0;
+    p.o_bytes = align256(rows * D * sizeof(float));
+    p.stage_at = p.o_bytes + align256(rows * 2 * sizeof(float));
+    const size_t blocks = static_cast<size_t>(NKV) * p.nblk;
+    p.pos_at = p.stage_at + blocks * 2 * kKeys * D * sizeof(uint16_t);
+    p.span_at = p.pos_at + align256(static_cast<size_t>(p.nblk) * kKeys * sizeof(int32_t));
+    p.ws_bytes = p.span_at + align256(static_cast<size_t>(p.nblk) * sizeof(int2));
+    return p;
+  }
   p.hw = NKV % 8 == 0 ? 8 : NKV % 4 == 0 ? 4 : NKV % 2 == 0 ? 2 : 1;
   p.ncg = p.mfma ? kCols : (NC < kGenOut / D ? NC : kGenOut / D);
   p.passes = (NC + p.ncg - 1) / p.ncg;
   p.ncp = p.passes * p.ncg;
-  const int nb = (TK + kKeys - 1) / kKeys;
   // default: 8 wavefronts per CU for the MFMA kernel, 2 workgroups of 4
   // wavefronts per CU for the generic one
   const long long target = p.mfma ? 8LL * device_cu_count() : 2LL * device_cu_count();
@@ -845,9 +1548,45 @@ PfPlan pf_plan(int B, int NQ, int TQ, int NKV, int D, int TK, int dtype, int num
   if (s > nb) s = nb;
   p.splits = s < 1 ? 1 : static_cast<int>(s);
   const size_t rows = static_cast<size_t>(B) * NKV * p.splits * p.ncp;
-  p.o_bytes = (rows * D * sizeof(float) + 255) & ~size_t(255);
+  p.o_bytes = align256(rows * D * sizeof(float));
   p.ws_bytes = p.o_bytes + rows * 2 * sizeof(float);
   return p;
+}
+
+// Stages the pages and runs the window kernels (a.part_* set).
+template <int D, typename E>
+int launch_pf_window(const PfPlan& p, const PfArgs& a, char* ws, bool f32_tab, void* out,
+                     hipStream_t stream) {
+  WinArgs w;
+  w.p = a;
+  const size_t blocks = static_cast<size_t>(a.NKV) * p.nblk;
+  w.k_blk = reinterpret_cast<uint16_t*>(ws + p.stage_at);
+  w.v_blk = w.k_blk + blocks * kKeys * D;
+  w.pos = reinterpret_cast<int32_t*>(ws + p.pos_at);
+  w.span = reinterpret_cast<int2*>(ws + p.span_at);
+  w.nblk = p.nblk;
+  w.R = a.B * a.NC;
+  w.row_tiles = p.row_tiles;
+  w.splits = p.splits;
+  w.work = a.NKV * p.row_tiles * p.splits;
+  w.per_xcd = (w.work + 7) / 8;
+  w.xcd_cus = device_cu_count() / 8;
+  w.scale = a.scale == 0.f ? 1.f : fabsf(a.scale_log2e);
+  w.q_keep = a.scale == 0.f ? 0u : 0xffffffffu;
+  w.q_flip = a.scale < 0.f ? 0x80008000u : 0u;
+  if (p.nblk > 0) {
+    const dim3 grid(static_cast<unsigned>(p.nblk) * a.NKV);
+    if (f32_tab) hipLaunchKernelGGL((pf_stage_kernel<D, E, EF32>), grid, dim3(256), 0, stream, w);
+    else hipLaunchKernelGGL((pf_stage_kernel<D, E, E>), grid, dim3(256), 0, stream, w);
+  }
+  hipLaunchKernelGGL((pf_window_kernel<D, E>), dim3(8u * static_cast<unsigned>(w.per_xcd)),
+                     dim3(kWinWaves * kWave), 0, stream, w, static_cast<uint16_t*>(out));
+  int rc = VOOM_LAUNCH_CHECK("position_free_attention: window launch");
+  if (rc || p.splits == 1) return rc;
+  const int rows = a.NKV * w.R;
+  hipLaunchKernelGGL((pf_window_combine_kernel<D, E>), dim3(static_cast<unsigned>((rows + 3) / 4)),
+                     dim3(256), 0, stream, w, static_cast<uint16_t*>(out), rows);
+  return VOOM_LAUNCH_CHECK("position_free_attention: combine launch");
 }
 
 bool pf_dtype_ok(int dt) {
@@ -933,8 +1672,10 @@ extern "C" int voom_position_free_attention(
   const int G = num_q_heads / num_kv_heads;
   const long long NC = static_cast<long long>(G) * num_queries;
   const long long segs = static_cast<long long>(batch) * num_kv_heads;
-  const long long nwork = segs * p.splits / (p.mfma ? p.hw : 1);
-  const long long grid_x = p.passes == 1 ? nwork : (nwork + 7) / 8 * 8 * p.passes;
+  const long long nwork = p.window ? static_cast<long long>(num_kv_heads) * p.row_tiles * p.splits
+                                   : segs * p.splits / (p.mfma ? p.hw : 1);
+  const long long grid_x =
+      p.window || p.passes == 1 ? nwork : (nwork + 7) / 8 * 8 * p.passes;
   VOOM_REQUIRE(NC < (1LL << 24) && grid_x < (1LL << 30) && segs * NC * (head_dim / 32) < (1LL << 31),
                "%s: grid too large", who);
 
@@ -969,16 +1710,22 @@ extern "C" int voom_position_free_attention(
   a.scale_log2e = scale * kLog2e;
   const dim3 grid(static_cast<unsigned>(grid_x));
   int rc;
+  if (p.window) {
+    char* ws = static_cast<char*>(workspace);
+    const bool f32_tab = table_dtype == VOOM_DTYPE_F32;
+    if (dtype == VOOM_DTYPE_BF16)
+      return head_dim == 128 ? launch_pf_window<128, EBf16>(p, a, ws, f32_tab, out, stream)
+                             : launch_pf_window<64, EBf16>(p, a, ws, f32_tab, out, stream);
+    return head_dim == 128 ? launch_pf_window<128, EF16>(p, a, ws, f32_tab, out, stream)
+                           : launch_pf_window<64, EF16>(p, a, ws, f32_tab, out, stream);
+  }
   if (p.mfma) {
     const dim3 block(static_cast<unsigned>(p.hw * kWave));
     const bool f32_tab = table_dtype == VOOM_DTYPE_F32;
-    if (head_dim == 128) {
-      if (f32_tab) launch_pf_attention<128, EF32>(p.hw, grid, block, stream, a);
-      else launch_pf_attention<128, EBf16>(p.hw, grid, block, stream, a);
-    } else {
-      if (f32_tab) launch_pf_attention<64, EF32>(p.hw, grid, block, stream, a);
-      else launch_pf_attention<64, EBf16>(p.hw, grid, block, stream, a);
-    }
+    if (dtype == VOOM_DTYPE_BF16)
+      launch_pf_attention_e<EBf16>(head_dim, f32_tab, p.hw, grid, block, stream, a);
+    else
+      launch_pf_attention_e<EF16>(head_dim, f32_tab, p.hw, grid, block, stream, a);
     rc = VOOM_LAUNCH_CHECK("position_free_attention: kernel launch");
   } else {
     const size_t lds = static_cast<size_t>(gen_lds(head_dim, p.ncg).words) * 4;
