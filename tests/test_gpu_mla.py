@@ -344,3 +344,36 @@ def test_head_gemv_writes_into_a_wider_row_and_rejects_bad_shapes():
         ops.head_gemv(x, torch.zeros((3, 48, 32), dtype=torch.bfloat16, device="cuda"))
     with pytest.raises(ValueError):
         ops.head_gemv(x[:, :2], packed)
+
+
+@pytest.mark.parametrize("batch,nr", [(1, 17), (1, 40), (1, 128), (1, 384), (1, 400), (3, 128),
+                                      (2, 193), (7, 33), (16, 17)])
+def test_merges_of_many_ranges(batch, nr):
+    """More than 16 ranges: merged in groups by several wavefronts while a
+    workgroup holds the groups' states (24: 1 x 384, 3 x 128, 7 x 33 and
+    16 x 17 lie on either side), else by one.  Both merging kernels give the
+    same bits, and the oracle's values (empty ranges among them)."""
+    print(f"[mla] merge of {nr} ranges, batch {batch}", flush=True)
+    ctx = [1500, 0, 700, 64, 65, 3, 900] + [130] * 9  # one of them empty
+    inp = synthetic.mla_decode_inputs(batch=batch, heads=64, ctx_lens=ctx[:batch])
+    check_latent(inp, num_ranges=nr, batches=[b for b in range(batch) if ctx[b]])
+    w_uk, w_uv_t = ops.split_kv_b(inp.kv_b, 64, inp.dn, inp.dv)
+    q_lat = ops.mla_absorb_query(inp.q_nope, inp.q_rope, w_uk)
+    wc, lse = ops.mla_latent_decode(q_lat, inp.lat_pool, inp.block_table, inp.ctx_lens,
+                                    scale=inp.scale, num_ranges=nr, return_lse=True)
+    _, wc2, lse2 = ops.mla_latent_decode_project(q_lat, inp.lat_pool, inp.block_table,
+                                                 inp.ctx_lens, w_uv_t, scale=inp.scale,
+                                                 num_ranges=nr, return_weighted_c=True,
+                                                 return_lse=True)
+    torch.cuda.synchronize()
+    assert torch.equal(wc.view(torch.int16), wc2.view(torch.int16)) and torch.equal(lse, lse2)
+    if batch > 1:  # the empty sequence
+        assert torch.all(wc[1] == 0) and torch.all(lse[1] == -float("inf"))
+
+
+@pytest.mark.parametrize("batch,heads,ctx", [(1, 128, 200), (5, 128, 1000), (9, 64, 450),
+                                             (1, 32, 3000)])
+def test_default_ranges_match_the_oracle(batch, heads, ctx):
+    print(f"[mla] default ranges batch={batch} heads={heads} ctx={ctx}", flush=True)
+    check_latent(synthetic.mla_decode_inputs(batch=batch, heads=heads,
+                                             ctx_lens=[max(1, ctx - 7 * b) for b in range(batch)]))

@@ -1150,20 +1150,21 @@ struct SmallRanges {
   f16x8 rows[kSmallRanges];
 };
 
+// Ranges r0 .. r0 + cnt - 1 (cnt <= kSmallRanges) of the NR of sequence b.
 __device__ __forceinline__ void load_small_ranges(const void* __restrict__ part_o16,
                                                   const float* __restrict__ part_ml, int b,
-                                                  int h, int H, int NR, int lane,
+                                                  int h, int H, int NR, int r0, int cnt, int lane,
                                                   SmallRanges& sr) {
+  const size_t first = static_cast<size_t>(b) * NR + r0;
   sr.st = f32x4{-INFINITY, 0.f, 0.f, 0.f};
-  if (lane < NR) {
-    sr.st = reinterpret_cast<const f32x4*>(part_ml)[(static_cast<size_t>(b) * NR + lane) * H + h];
+  if (lane < cnt) {
+    sr.st = reinterpret_cast<const f32x4*>(part_ml)[(first + lane) * H + h];
   }
 #pragma unroll
   for (int r = 0; r < kSmallRanges; ++r) {
-    const int rr = r < NR ? r : NR - 1;
-    sr.rows[r] = *reinterpret_cast<const f16x8*>(
-        static_cast<const _Float16*>(part_o16) +
-        ((static_cast<size_t>(b) * NR + rr) * H + h) * kC + lane * kDPL);
+    const int rr = r < cnt ? r : cnt - 1;
+    sr.rows[r] = *reinterpret_cast<const f16x8*>(static_cast<const _Float16*>(part_o16) +
+                                                 ((first + rr) * H + h) * kC + lane * kDPL);
   }
 }
 
@@ -1189,6 +1190,63 @@ __device__ __forceinline__ void combine_small_ranges(const SmallRanges& sr, int 
                     static_cast<float>(x[3])} * wk;
     acc[1] += f32x4{static_cast<float>(x[4]), static_cast<float>(x[5]), static_cast<float>(x[6]),
                     static_cast<float>(x[7])} * wk;
+  }
+}
+
+// More than kSmallRanges ranges (few sequences, which leave many ranges each):
+// groups of kSmallRanges are merged by as many wavefronts, each in its one
+// memory round trip, and the groups' states meet in LDS in group order.  One
+// wavefront per sequence took a round trip per eight ranges (1 sequence, 128
+// ranges: 18 of 38 us).  The rule depends on (B, NR) only and both merging
+// kernels use it, so they give the same bits.
+constexpr int kMaxStates = 24;  // group states a workgroup of the fused merge can hold
+__host__ __device__ __forceinline__ int range_groups(int NR) {
+  return (NR + kSmallRanges - 1) / kSmallRanges;
+}
+__host__ __device__ __forceinline__ bool merges_in_groups(int B, int NR) {
+  return NR > kSmallRanges && static_cast<long long>(B) * range_groups(NR) <= kMaxStates;
+}
+struct GroupState {
+  float o[kC];  // sum of the group's weighted rows, relative to M
+  float M, L;
+};
+__device__ __forceinline__ int group_count(int NR, int group) {
+  const int left = NR - group * kSmallRanges;
+  return left < kSmallRanges ? left : kSmallRanges;
+}
+__device__ __forceinline__ void load_group(const void* __restrict__ part_o16,
+                                           const float* __restrict__ part_ml, int b, int h, int H,
+                                           int NR, int group, int lane, SmallRanges& sr) {
+  load_small_ranges(part_o16, part_ml, b, h, H, NR, group * kSmallRanges, group_count(NR, group),
+                    lane, sr);
+}
+__device__ __forceinline__ void store_group(const SmallRanges& sr, int NR, int group, int lane,
+                                            GroupState* st) {
+  f32x4 acc[kDPL / 4];
+  float M, L;
+  combine_small_ranges(sr, group_count(NR, group), lane, acc, M, L);
+#pragma unroll
+  for (int c = 0; c < kDPL / 4; ++c)
+    *reinterpret_cast<f32x4*>(&st->o[lane * kDPL + 4 * c]) = acc[c];
+  if (lane == 0) {
+    st->M = M;
+    st->L = L;
+  }
+}
+__device__ __forceinline__ void combine_groups(const GroupState* st, int groups, int lane,
+                                               f32x4 (&acc)[kDPL / 4], float& M, float& L) {
+  M = -INFINITY;
+  for (int g = 0; g < groups; ++g) M = fmaxf(M, st[g].M);
+  L = 0.f;
+#pragma unroll
+  for (int c = 0; c < kDPL / 4; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (M == -INFINITY) return;
+  for (int g = 0; g < groups; ++g) {
+    const float wt = st[g].M == -INFINITY ? 0.f : fast_exp2(st[g].M - M);
+    L += st[g].L * wt;
+#pragma unroll
+    for (int c = 0; c < kDPL / 4; ++c)
+      acc[c] += *reinterpret_cast<const f32x4*>(&st[g].o[lane * kDPL + 4 * c]) * wt;
   }
 }
 
@@ -1220,11 +1278,39 @@ __global__ __launch_bounds__(kThreads) void mla_reduce_kernel(
   float M, L;
   if (F16 && NR <= kSmallRanges) {
     SmallRanges sr;
-    load_small_ranges(part_o, part_ml, b, h, H, NR, lane, sr);
+    load_small_ranges(part_o, part_ml, b, h, H, NR, 0, NR, lane, sr);
     combine_small_ranges(sr, NR, lane, acc, M, L);
   } else {
     merge_ranges<F16>(part_o, part_ml, b, h, H, NR, lane, acc, M, L);
   }
+  *reinterpret_cast<u32x4*>(out + static_cast<size_t>(task) * kC + lane * kDPL) =
+      merged_row_bf16(acc, L);
+  if (lse_out != nullptr && lane == 0) lse_out[task] = merged_lse(M, L);
+}
+
+// mla_reduce_kernel<true> where merges_in_groups: one workgroup of eight
+// wavefronts per (sequence, head).
+constexpr int kRgThreads = 512;
+__global__ __launch_bounds__(kRgThreads) void mla_reduce_groups_kernel(
+    const void* __restrict__ part_o, const float* __restrict__ part_ml,
+    uint16_t* __restrict__ out, float* __restrict__ lse_out, int B, int H, int NR) {
+  __shared__ __attribute__((aligned(16))) GroupState st[kMaxStates];
+  const int lane = threadIdx.x & 63;
+  const int w = uniform(threadIdx.x >> 6);
+  const int task = blockIdx.x;
+  const int b = task / H;
+  const int h = task - b * H;
+  const int groups = range_groups(NR);
+  for (int g = w; g < groups; g += kRgThreads / kWave) {
+    SmallRanges sr;
+    load_group(part_o, part_ml, b, h, H, NR, g, lane, sr);
+    store_group(sr, NR, g, lane, &st[g]);
+  }
+  lds_barrier();
+  if (w != 0) return;
+  f32x4 acc[kDPL / 4];
+  float M, L;
+  combine_groups(st, groups, lane, acc, M, L);
   *reinterpret_cast<u32x4*>(out + static_cast<size_t>(task) * kC + lane * kDPL) =
       merged_row_bf16(acc, L);
   if (lse_out != nullptr && lane == 0) lse_out[task] = merged_lse(M, L);
@@ -1238,17 +1324,20 @@ __global__ __launch_bounds__(kThreads) void mla_reduce_kernel(
 // voom_mla_head_gemv, dv <= 128: at most 128 KiB) streams into LDS from the
 // first instruction on, beside the partial rows the merge reads, so one
 // launch replaces the merge and the projection's weight stream.  Eight
-// wavefronts: wavefront w merges sequences w, w + 8, then projects column
-// tiles w, w + 8.
+// wavefronts: wavefront w merges sequences w, w + 8 (or, with many ranges,
+// their groups of ranges), then projects column tiles w, w + 8.
 constexpr int kRpMaxTiles = 8;                 // dv <= 128
+constexpr int kRpPartTiles = kRpMaxTiles / 2;  // column tiles of one workgroup (two parts)
 constexpr int kRpSteps = kC / kHgStep;         // 16 k-steps over the 512 latent dims
 constexpr int kRpThreads = 512;                // 8 wavefronts: one per sequence, one per tile
+template <bool GROUPED>  // merges_in_groups(B, NR): apart, so that the usual merge keeps its registers
 __global__ __launch_bounds__(kRpThreads) void mla_reduce_project_kernel(
     const void* __restrict__ part_o16, const float* __restrict__ part_ml,
     const uint16_t* __restrict__ w_uv, uint16_t* __restrict__ y, uint16_t* __restrict__ wc_out,
     float* __restrict__ lse_out, int B, int H, int NR, int DV, int NT, int splits) {
-  __shared__ __attribute__((aligned(16))) uint16_t wl[kRpMaxTiles * kRpSteps * 512];
+  __shared__ __attribute__((aligned(16))) uint16_t wl[kRpPartTiles * kRpSteps * 512];
   __shared__ __attribute__((aligned(16))) uint16_t wcs[16][kC + 8];
+  __shared__ __attribute__((aligned(16))) GroupState states[GROUPED ? kMaxStates : 1];
   // workgroups h + H part (same XCD for every part of a head when H % 8 == 0,
   // so the parts' reads of the head's partial rows meet in one L2) split the
   // head's column tiles; each merges all rows, part 0 writes weighted_c / lse
@@ -1264,9 +1353,12 @@ __global__ __launch_bounds__(kRpThreads) void mla_reduce_project_kernel(
   // ranges, every partial row), then the weight stream: the merge waits only
   // for its own loads, which the wait counter drains in issue order.
   const int bw = w < B ? w : 0;  // wavefronts past B merge row 0 and keep nothing
-  const bool small = NR <= kSmallRanges;
+  const bool small = !GROUPED && NR <= kSmallRanges;
+  const int groups = range_groups(NR);
   SmallRanges sr;
-  if (small) load_small_ranges(part_o16, part_ml, bw, h, H, NR, lane, sr);
+  if (small) load_small_ranges(part_o16, part_ml, bw, h, H, NR, 0, NR, lane, sr);
+  if (GROUPED && w < B * groups)
+    load_group(part_o16, part_ml, w / groups, h, H, NR, w % groups, lane, sr);
   {
     // this part's tiles: blocks nt_lo * 16 .. nt_hi * 16 (1 KiB each) of the head
     const int blocks = (nt_hi - nt_lo) * kRpSteps;
@@ -1278,10 +1370,19 @@ __global__ __launch_bounds__(kRpThreads) void mla_reduce_project_kernel(
                                                0, 0, 0);
     }
   }
+  if constexpr (GROUPED) {
+    for (int i = w; i < B * groups; i += kWaves) {
+      if (i != w) load_group(part_o16, part_ml, i / groups, h, H, NR, i % groups, lane, sr);
+      store_group(sr, NR, i % groups, lane, &states[i]);
+    }
+    lds_barrier();
+  }
   for (int b = w; b < B; b += kWaves) {
     f32x4 acc[kDPL / 4];
     float M, L;
-    if (small && b == w) {
+    if constexpr (GROUPED) {
+      combine_groups(states + b * groups, groups, lane, acc, M, L);
+    } else if (small && b == w) {
       combine_small_ranges(sr, NR, lane, acc, M, L);  // the rows loaded at kernel start
     } else {
       merge_ranges<true>(part_o16, part_ml, b, h, H, NR, lane, acc, M, L);
@@ -1323,10 +1424,43 @@ __global__ __launch_bounds__(kRpThreads) void mla_reduce_project_kernel(
 // Heads per workgroup for a head count: 64 when it divides, else 32.
 int heads_per_group(int H) { return H % 64 == 0 ? 64 : 32; }
 
+// The most ranges per sequence that leave every workgroup a CU of its own: its
+// LDS tiles fill one, so a 257th workgroup doubles the launch's time (5
+// sequences of 16,384 tokens, 128 heads: 26 ranges 69 us, 25 ranges 50 us).
 int default_ranges(int B, int H) {
-  const int wgs_per_range = B * (H / heads_per_group(H));
-  int nr = (device_cu_count() + wgs_per_range - 1) / wgs_per_range;
+  const int nr = device_cu_count() / (B * (H / heads_per_group(H)));
   return nr < 1 ? 1 : nr;
+}
+
+// Ranges of a dense call over tables of at most `tiles` 64-token tiles: of the
+// counts that default_ranges allows, the one with the least of
+//   1.75 us per tile of a range (they run one after the other),
+//   0.03 us per workgroup for its partial rows, written and read back,
+//   1 us per round trip of the grouped merge past 16 ranges, 0.25 us per range
+//   where one wavefront merges them (0.1 us with 32-head groups, fp32 rows).
+// Fitted to sweeps over 1-16 sequences of 200-65,536 tokens and 32-128 heads;
+// default_ranges alone, before: 128 heads, 1 sequence of 200 / 1,000 / 16,384
+// tokens 36 / 35 / 38 us, now 20 / 20 / 29; 6 of 8,000: 51, now 39; 64 heads, 1 of
+// 1,000: 44, now 18.
+int dense_ranges(int B, int H, long long tiles) {
+  const int hg = heads_per_group(H);
+  const int most = default_ranges(B, H);
+  const double wgs = static_cast<double>(B) * (H / hg);
+  int best = most;
+  double least = 1e30;
+  const long long p0 = (tiles + most - 1) / most;
+  for (long long p = p0; p < p0 + 16 && p <= tiles; ++p) {
+    const int nr = static_cast<int>((tiles + p - 1) / p);
+    double cost = 1.75 * static_cast<double>(p) + 0.03 * wgs * nr;
+    if (hg != 64) cost += 0.1 * nr;
+    else if (merges_in_groups(B, nr)) cost += (B * range_groups(nr) + 7) / 8;
+    else if (nr > kSmallRanges) cost += 0.25 * nr;
+    if (cost < least) {
+      least = cost;
+      best = nr;
+    }
+  }
+  return best;
 }
 
 // Latent kernel (dense or sparse) and the range reduce.
@@ -1349,7 +1483,11 @@ int launch_mla(const MlaArgs& a, int hg, bool sparse, long long grid, uint16_t* 
   int rc = VOOM_LAUNCH_CHECK("mla: latent kernel launch");
   if (rc) return rc;
   const unsigned red_grid = static_cast<unsigned>((a.B * a.H + 3) / 4);
-  if (hg == 64) {
+  if (hg == 64 && merges_in_groups(a.B, a.NR)) {
+    hipLaunchKernelGGL(mla_reduce_groups_kernel, dim3(static_cast<unsigned>(a.B * a.H)),
+                       dim3(kRgThreads), 0, stream, static_cast<const void*>(a.part_o16), a.part_ml,
+                       out, lse_out, a.B, a.H, a.NR);
+  } else if (hg == 64) {
     hipLaunchKernelGGL(mla_reduce_kernel<true>, dim3(red_grid), dim3(kThreads), 0, stream,
                        static_cast<const void*>(a.part_o16), a.part_ml, out, lse_out, a.B, a.H, a.NR);
   } else {
@@ -1370,8 +1508,10 @@ int launch_mla_project(const MlaArgs& a, long long grid, const void* w_uv_packed
   // two parts per head when there are at least two column tiles: twice the
   // workgroups for the weight stream
   const int splits = nt >= 2 ? 2 : 1;
-  hipLaunchKernelGGL(mla_reduce_project_kernel, dim3(static_cast<unsigned>(a.H * splits)),
-                     dim3(kRpThreads), 0, stream, static_cast<const void*>(a.part_o16), a.part_ml,
+  auto* kernel = merges_in_groups(a.B, a.NR) ? mla_reduce_project_kernel<true>
+                                             : mla_reduce_project_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(a.H * splits)), dim3(kRpThreads), 0,
+                     stream, static_cast<const void*>(a.part_o16), a.part_ml,
                      static_cast<const uint16_t*>(w_uv_packed), static_cast<uint16_t*>(y), wc_out,
                      lse_out, a.B, a.H, a.NR, dv, nt, splits);
   return VOOM_LAUNCH_CHECK("mla: merge + projection kernel launch");
@@ -1617,7 +1757,9 @@ int prepare_dense(const char* who, const void* q_lat, const void* lat_pool,
                static_cast<double>(scale));
   VOOM_REQUIRE(static_cast<long long>(max_pages) * page_tokens < (1LL << 30),
                "%s: table capacity too large", who);
-  if (num_ranges <= 0) num_ranges = default_ranges(batch, num_heads);
+  if (num_ranges <= 0)
+    num_ranges = dense_ranges(batch, num_heads,
+                              (static_cast<long long>(max_pages) * page_tokens + kTile - 1) / kTile);
   const size_t need = voom_mla_workspace_bytes(batch, num_heads, num_ranges);
   VOOM_REQUIRE(ws_bytes >= need, "%s: workspace %zu bytes < required %zu", who, ws_bytes, need);
   VOOM_REQUIRE(reinterpret_cast<uintptr_t>(q_lat) % 16 == 0 &&
