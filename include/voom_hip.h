@@ -175,6 +175,19 @@ int voom_mla_absorb_query(const void* q_nope, const void* q_rope, const void* w_
                           void* q_lat, int batch, int num_heads, int dn, int c_dim, int rope_dim,
                           hipStream_t stream);
 
+/* The per-head products of voom_mla_head_gemv / voom_mla_absorb_query for many
+ * rows (the queries of a prompt), bit for bit: y[row, h, :n] = x[row, h, :k] .
+ * w[h], then, with tail, y[row, h, n : n + tail_cols] = tail[row, h].  Row = (batch
+ * entry, token); x and tail are addressed through element strides per batch
+ * entry, token and head (multiples of 8), y is [batch * tokens, heads, y_stride]
+ * bf16.  k a multiple of 8 up to 512, n one of 4 (of 8 with a tail). */
+int voom_mla_head_rows(const void* x, const void* tail, const void* w_packed, void* y, int batch,
+                       int tokens, int num_heads, int k, int n, long long x_batch,
+                       long long x_token, long long x_head, int tail_cols, long long tail_batch,
+                       long long tail_token, long long tail_head, int y_stride,
+                       hipStream_t stream);
+
+
 /* Bytes of the packed form of per-head weights w [num_heads, k, n] bf16
  * (k and n padded to multiples of 32 and 16). */
 size_t voom_mla_head_weights_bytes(int num_heads, int k, int n);

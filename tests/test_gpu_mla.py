@@ -377,3 +377,32 @@ def test_default_ranges_match_the_oracle(batch, heads, ctx):
     print(f"[mla] default ranges batch={batch} heads={heads} ctx={ctx}", flush=True)
     check_latent(synthetic.mla_decode_inputs(batch=batch, heads=heads,
                                              ctx_lens=[max(1, ctx - 7 * b) for b in range(batch)]))
+
+
+@pytest.mark.parametrize("B,L,H,K,N,dr", [(1, 17, 128, 128, 512, 64), (2, 30, 5, 40, 64, 8),
+                                          (1, 301, 4, 512, 128, 0), (3, 11, 2, 8, 24, 0),
+                                          (1, 33, 3, 200, 512, 64), (1, 1000, 2, 128, 512, 64)])
+def test_products_of_many_rows_have_the_decode_bits(B, L, H, K, N, dr):
+    """voom_mla_head_rows against 16 rows at a time of the decode kernels, from
+    contiguous, token-major and misaligned queries."""
+    print(f"[mla] head rows B={B} L={L} H={H} K={K} N={N} dr={dr}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(L + H + K)
+    x = torch.randn((B, H, L, K), generator=g, device="cuda").to(torch.bfloat16)
+    w = ops.pack_head_weights((torch.randn((H, K, N), generator=g, device="cuda") * 0.05).to(
+        torch.bfloat16))
+    rows = x.permute(0, 2, 1, 3).reshape(B * L, H, K).contiguous()
+    if dr == 0:
+        ref = torch.cat([ops.head_gemv(rows[i:i + 16], w) for i in range(0, B * L, 16)])
+        got = [ops.mla_project_rows(rows, w)]
+    else:
+        t = torch.randn((B, H, L, dr), generator=g, device="cuda").to(torch.bfloat16)
+        trows = t.permute(0, 2, 1, 3).reshape(B * L, H, dr).contiguous()
+        ref = torch.cat([ops.mla_absorb_query(rows[i:i + 16], trows[i:i + 16], w)
+                         for i in range(0, B * L, 16)])
+        odd = torch.empty(x.numel() + 1, dtype=x.dtype, device="cuda")[1:].view(x.shape).copy_(x)
+        token_major = x.transpose(1, 2).contiguous().transpose(1, 2)
+        got = [ops.mla_absorb_query_tokens(q, r, w) for q, r in
+               ((x, t), (token_major, t.transpose(1, 2).contiguous().transpose(1, 2)), (odd, t))]
+    torch.cuda.synchronize()
+    for y in got:
+        assert torch.equal(y.view(torch.int16), ref.view(torch.int16))

@@ -11,7 +11,7 @@ from __future__ import annotations
 import atexit
 import ctypes
 import threading
-from ctypes import c_float, c_int, c_size_t, c_void_p
+from ctypes import c_float, c_int, c_longlong, c_size_t, c_void_p
 
 from ._build import LIB_PATH
 
@@ -68,6 +68,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "voom_mla_head_weights_bytes": (c_size_t, [c_int, c_int, c_int]),
     "voom_mla_pack_head_weights": (c_int, [_P, _P, c_int, c_int, c_int, _P]),
     "voom_mla_absorb_query": (c_int, [_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, _P]),
+    "voom_mla_head_rows": (c_int, [_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_longlong,
+                                   c_longlong, c_longlong, c_int, c_longlong, c_longlong,
+                                   c_longlong, c_int, _P]),
     "voom_lm_head_argmax": (c_int, [_P, _P, _P, c_float, _P, c_int, c_int, _P, c_size_t, _P, _P,
                                     _P]),
     "voom_add_rms_norm_gemv": (c_int, [_P, _P, _P, c_float, _P, _P, _P, c_int, c_int, c_int,

@@ -2047,8 +2047,8 @@ class PagedKVCache:
         cast points (fp32 scores, bf16 P, bf16 weighted_c; :157-164).  As in
         ``attend_prefill``, every query row becomes its own entry of the paged
         latent kernel -- the same block-table row with the context cut at its
-        own position + 1 -- and the absorption products run on the decode
-        kernels, 16 rows per launch, so L = 1 gives ``attend_mla``'s bits.
+        own position + 1 -- and the absorption products give the decode
+        kernels' bits, so L = 1 gives ``attend_mla``'s.
         Spilled pages of the layer are made resident first.  Returns the
         per-head output [B, H, L, dv] (and weighted_c [B, H, L, 512]).
         """
@@ -2068,13 +2068,21 @@ class PagedKVCache:
         pool = self._pool(layer)
         w_uk = ops.pack_head_weights(w_uk)
         w_uv = ops.pack_head_weights(w_uv_t)
+        if w_uk.n != 512:  # weighted_c's width, written straight into wc below
+            raise ValueError(f"W_UK must be [H, dn, 512], got {w_uk.shape}")
         R = B * L
-        rows_n = q_nope.permute(0, 2, 1, 3).reshape(R, H, dn).contiguous()
-        rows_r = q_rope.permute(0, 2, 1, 3).reshape(R, H, dr).contiguous()
-        q_lat = torch.empty((R, H, w_uk.n + dr), dtype=torch.bfloat16, device=self.device)
-        for r0 in range(0, R, 16):  # the head products take at most 16 rows
-            r1 = min(R, r0 + 16)
-            q_lat[r0:r1] = ops.mla_absorb_query(rows_n[r0:r1], rows_r[r0:r1], w_uk)
+        # up to 16 rows are one launch of the decode step's products; more keep
+        # the weights in registers and stream the rows past them
+        many = R > 16 and ops.head_rows_supported(w_uk, dr) and ops.head_rows_supported(w_uv)
+        if many:
+            q_lat = ops.mla_absorb_query_tokens(q_nope, q_rope, w_uk)
+        else:
+            rows_n = q_nope.permute(0, 2, 1, 3).reshape(R, H, dn).contiguous()
+            rows_r = q_rope.permute(0, 2, 1, 3).reshape(R, H, dr).contiguous()
+            q_lat = torch.empty((R, H, w_uk.n + dr), dtype=torch.bfloat16, device=self.device)
+            for r0 in range(0, R, 16):  # the head products take at most 16 rows
+                r1 = min(R, r0 + 16)
+                q_lat[r0:r1] = ops.mla_absorb_query(rows_n[r0:r1], rows_r[r0:r1], w_uk)
         table = self._tables[layer].repeat_interleave(L, dim=0)
         ctx = (torch.arange(S - L + 1, S + 1, dtype=torch.int32, device=self.device)
                .repeat(B))
@@ -2082,12 +2090,15 @@ class PagedKVCache:
         step = 256  # query rows per latent launch (bounds the range partials)
         for r0 in range(0, R, step):
             r1 = min(R, r0 + step)
-            wc[r0:r1] = ops.mla_latent_decode(q_lat[r0:r1], pool.lat, table[r0:r1].contiguous(),
-                                              ctx[r0:r1].contiguous(), scale=scale)
-        out = torch.empty((R, H, w_uv.n), dtype=torch.bfloat16, device=self.device)
-        for r0 in range(0, R, 16):
-            r1 = min(R, r0 + 16)
-            out[r0:r1] = ops.mla_project_out(wc[r0:r1], w_uv)
+            ops.mla_latent_decode(q_lat[r0:r1], pool.lat, table[r0:r1], ctx[r0:r1], scale=scale,
+                                  out=wc[r0:r1])
+        if many:
+            out = ops.mla_project_rows(wc, w_uv)
+        else:
+            out = torch.empty((R, H, w_uv.n), dtype=torch.bfloat16, device=self.device)
+            for r0 in range(0, R, 16):
+                r1 = min(R, r0 + 16)
+                out[r0:r1] = ops.mla_project_out(wc[r0:r1], w_uv)
         out = out.reshape(B, L, H, w_uv.n).permute(0, 2, 1, 3)
         if return_weighted_c:
             return out, wc.reshape(B, L, H, w_uk.n).permute(0, 2, 1, 3)

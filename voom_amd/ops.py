@@ -924,6 +924,56 @@ def mla_absorb_query(q_nope: torch.Tensor, q_rope: torch.Tensor, w_uk):
     return q_lat
 
 
+def head_rows_supported(w: HeadWeights, tail: int = 0) -> bool:
+    """Whether voom_mla_head_rows takes these weights (and a tail of that many
+    columns): whole 16-byte pieces, K within a wavefront's registers."""
+    return (w.k % 8 == 0 and 8 <= w.k <= 512 and w.n % (8 if tail else 4) == 0
+            and (tail == 0 or tail % 8 == 0))
+
+
+def _token_rows(t: torch.Tensor) -> torch.Tensor:
+    """[B, H, L, D] as voom_mla_head_rows reads it: unit stride in D, the others
+    and the start 16-byte aligned (a copy where they are not)."""
+    if t.stride(3) != 1 or any(t.stride(i) % 8 for i in range(3)) or t.data_ptr() % 16:
+        t = t.contiguous()
+        if t.data_ptr() % 16:
+            t = t.clone()
+    return t
+
+
+def mla_absorb_query_tokens(q_nope: torch.Tensor, q_rope: torch.Tensor,
+                            w_uk: HeadWeights) -> torch.Tensor:
+    """``mla_absorb_query`` of every token of a window, with the same bits:
+    q_nope [B, H, L, dn], q_rope [B, H, L, dr] bf16 -> q_lat [B * L, H, C + dr].
+    dn a multiple of 8 up to 512, C and dr multiples of 8."""
+    _require(q_nope.is_cuda and q_rope.device == q_nope.device == w_uk.packed.device,
+             "q and W_UK must be on one ROCm device")
+    _require(q_nope.dtype == q_rope.dtype == torch.bfloat16, "bf16 q_nope and q_rope")
+    B, H, L, dn = q_nope.shape
+    dr = q_rope.shape[-1]
+    _require(w_uk.heads == H and w_uk.k == dn, "W_UK must be [H, dn, C] for q_nope")
+    q_nope, q_rope = _token_rows(q_nope), _token_rows(q_rope)
+    q_lat = torch.empty((B * L, H, w_uk.n + dr), dtype=torch.bfloat16, device=q_nope.device)
+    sx, st = q_nope.stride(), q_rope.stride()
+    _lib.call("voom_mla_head_rows", _ptr(q_nope), _ptr(q_rope), _ptr(w_uk.packed), _ptr(q_lat), B,
+              L, H, dn, w_uk.n, sx[0], sx[2], sx[1], dr, st[0], st[2], st[1], w_uk.n + dr,
+              _stream(None))
+    return q_lat
+
+
+def mla_project_rows(wc: torch.Tensor, w_uv: HeadWeights) -> torch.Tensor:
+    """``mla_project_out`` of any number of rows, with the same bits: weighted_c
+    [R, H, C] bf16 -> [R, H, dv] (C a multiple of 8 up to 512, dv one of 4)."""
+    _require_device(wc, w_uv.packed)
+    _require(wc.dtype == torch.bfloat16 and wc.dim() == 3, "bf16 weighted_c [R, H, C]")
+    R, H, C = wc.shape
+    _require(w_uv.heads == H and w_uv.k == C, "W_UV^T must be [H, C, dv] for weighted_c")
+    out = torch.empty((R, H, w_uv.n), dtype=torch.bfloat16, device=wc.device)
+    _lib.call("voom_mla_head_rows", _ptr(wc), None, _ptr(w_uv.packed), _ptr(out), 1, R, H, C,
+              w_uv.n, R * H * C, H * C, C, 0, 0, 0, 0, w_uv.n, _stream(None))
+    return out
+
+
 def mla_project_out(wc: torch.Tensor, w_uv_t) -> torch.Tensor:
     """weighted_c [B, H, 512] . W_UV -> [B, H, dv] (runtime/glm.py:200-202)."""
     return head_gemv(wc, w_uv_t)
