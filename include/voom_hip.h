@@ -442,6 +442,33 @@ int voom_qkv_rope_append(const void* w_qkv, const void* x, const void* delta,
                          int num_kv_heads, int head_dim, int k, int page_tokens, int max_pages,
                          int num_slots, int rope_rows, hipStream_t stream);
 
+/* voom_linear_rows: voom_gemv_bf16 for `rows` rows at once (a prompt, a batch of
+ * tokens): x [rows, k], y [rows, n], k a multiple of 32 up to 2048, n of 8, fp32
+ * sums on the matrix cores.
+ *
+ * voom_norm_swiglu_rows: the same behind the residual add + RMSNorm of
+ * voom_add_rms_norm_gemv (ln_weight [k]; delta and x_out [rows, k] optional) and
+ * followed by SwiGLU, weight the fused [gate; up] [2n, k].
+ *
+ * voom_qkv_rope_append_rows: with that residual add + RMSNorm, `seq` tokens of each
+ * of `batch` sequences through the fused qkv projection, RoPE with the fp32 rows
+ * cos_table / sin_table [seq, head_dim] and the page write of k and v at positions
+ * start .. start + seq - 1 through block_table [batch, max_pages]; q [batch,
+ * num_q_heads, seq, head_dim] out.  head_dim a multiple of 32.  The dense block's
+ * projections of a prompt, runtime/layer_runner.py:73-103 and :188. */
+int voom_linear_rows(const void* x, const void* weight, void* y, int rows, int n, int k,
+                     hipStream_t stream);
+int voom_norm_swiglu_rows(const void* x, const void* delta, const void* ln_weight, float eps,
+                          void* x_out, const void* weight, void* y, int rows, int n, int k,
+                          hipStream_t stream);
+int voom_qkv_rope_append_rows(const void* w_qkv, const void* x, const void* delta,
+                              const void* ln_weight, float eps, void* x_out,
+                              const float* cos_table, const float* sin_table, void* q,
+                              void* k_pool, void* v_pool, const int32_t* block_table, int batch,
+                              int seq, int start, int num_q_heads, int num_kv_heads, int head_dim,
+                              int k, int page_tokens, int max_pages, int num_slots,
+                              hipStream_t stream);
+
 /* ---------------------------------------------------------------------------
  * Page writes and reads.
  *

@@ -75,6 +75,11 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
                                     _P]),
     "voom_add_rms_norm_gemv": (c_int, [_P, _P, _P, c_float, _P, _P, _P, c_int, c_int, c_int,
                                        _P]),
+    "voom_linear_rows": (c_int, [_P, _P, _P, c_int, c_int, c_int, _P]),
+    "voom_norm_swiglu_rows": (c_int, [_P, _P, _P, c_float, _P, _P, _P, c_int, c_int, c_int, _P]),
+    "voom_qkv_rope_append_rows": (c_int, [_P, _P, _P, _P, c_float, _P, _P, _P, _P, _P, _P, _P,
+                                          c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
+                                          c_int, c_int, _P]),
     "voom_position_free_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int,
                                                       c_int, c_int]),
     "voom_position_free_attention": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, c_size_t,

@@ -17,22 +17,24 @@ namespace {
 
 constexpr int kRowThreads = 256;
 
+// bf16(a + d) of two 16-byte chunks.
+__device__ __forceinline__ u32x4 sum_chunks(u32x4 a, u32x4 d) {
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const float lo = bf2f(static_cast<uint16_t>(a[w] & 0xffffu)) +
+                     bf2f(static_cast<uint16_t>(d[w] & 0xffffu));
+    const float hi = bf2f(static_cast<uint16_t>(a[w] >> 16)) +
+                     bf2f(static_cast<uint16_t>(d[w] >> 16));
+    a[w] = pack_bf16x2(lo, hi);
+  }
+  return a;
+}
+
 // 16-byte chunk at col of bf16(x + delta) (of x alone without delta).
 __device__ __forceinline__ u32x4 add_chunk(const uint16_t* __restrict__ x,
                                            const uint16_t* __restrict__ delta, int col) {
-  u32x4 a = *reinterpret_cast<const u32x4*>(x + col);
-  if (delta) {
-    const u32x4 d = *reinterpret_cast<const u32x4*>(delta + col);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const float lo = bf2f(static_cast<uint16_t>(a[w] & 0xffffu)) +
-                       bf2f(static_cast<uint16_t>(d[w] & 0xffffu));
-      const float hi = bf2f(static_cast<uint16_t>(a[w] >> 16)) +
-                       bf2f(static_cast<uint16_t>(d[w] >> 16));
-      a[w] = pack_bf16x2(lo, hi);
-    }
-  }
-  return a;
+  const u32x4 a = *reinterpret_cast<const u32x4*>(x + col);
+  return delta ? sum_chunks(a, *reinterpret_cast<const u32x4*>(delta + col)) : a;
 }
 
 // Sum of squares of one chunk's 8 values added to ss, in element order with
@@ -556,6 +558,313 @@ int launch_gemv(const uint16_t* w, const uint16_t* x, const uint16_t* delta, con
   return VOOM_LAUNCH_CHECK("gemv: kernel launch");
 }
 
+// Projections of several rows (a prompt, a batch of tokens): y = x . W^T with
+// the decode kernels' fusions around it -- the residual add + RMSNorm of the
+// rows in front and SwiGLU (kSwiglu) or RoPE and the page write of k and v
+// (kRope) behind, or neither (kPlain).  A prompt of a small model is bound by its
+// launches, not by its sums (a 512-row projection with k 576 and n 960 is 0.2 us
+// of matrix work), so the aim is few launches, each one memory round trip deep:
+//   a workgroup takes 32 rows and NW wavefronts of 16-column weight tiles (two
+//   tiles for the pairs of SwiGLU and RoPE).  Its rows and each wavefront's first
+//   2 SC k-steps of weights are put in flight together, straight into registers;
+//   the rows are normed, LPR lanes a row, and left in LDS, and the MFMAs take the
+//   weights as A and the rows as B: a lane ends with four adjacent columns of one
+//   row, and a pair's two halves are in one lane.
+// The rows are prepared again by each column group; that is 37 KB of reads that
+// hit L2, against a launch.  Column groups go round the XCDs, so each weight
+// crosses into one L2 only.  512 rows (k 576): qkv with its norm, RoPE and page
+// write 13.1 us, gate/up with norm and SwiGLU 15.8, 576 columns 6.7, and down
+// (k 1536) 11.2; as separate launches around library products a 30-layer prompt of
+// 512 tokens took 5.6 ms, so 2.3, and one of 64 tokens 5.2, so 2.0, both then
+// bound by the host.
+enum RowsMode { kPlain, kSwiglu, kRope };
+constexpr int kRowsTile = 32;   // rows of one workgroup
+constexpr int kRowsUnit = 256;  // k of one LDS size class
+
+struct RowsArgs {
+  const uint16_t* x;
+  const uint16_t* delta;
+  const uint16_t* ln;
+  uint16_t* x_out;
+  const uint16_t* w;
+  uint16_t* y;  // q in kRope
+  int rows, n, k;
+  int tiles;       // 16-column tiles (kSwiglu, kRope: tile pairs)
+  int groups;      // column groups: of NW tiles
+  int row_groups;  // groups of kRowsTile rows
+  float eps;
+  // kRope
+  const float* cos_t;
+  const float* sin_t;
+  uint16_t* k_pool;
+  uint16_t* v_pool;
+  const int32_t* table;
+  int L, start, nq, nkv, hd, pt_shift, max_pages, num_slots;
+};
+
+// Sum over each aligned group of LPR (8 or 16) lanes, the same value in all.
+template <int LPR>
+__device__ __forceinline__ float group_sum(float v) {
+  v += dpp_move<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+  v += dpp_move<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+  v += dpp_move<0x141>(v);  // row_half_mirror
+  if (LPR == 16) v += dpp_move<0x140>(v);  // row_mirror
+  return v;
+}
+
+__device__ __forceinline__ uint16_t swiglu_bf16(float gate, float up) {
+  const float g = bf2f(f2bf(gate));
+  const float s = bf2f(f2bf(g / (1.f + expf(-g))));
+  return f2bf(s * bf2f(f2bf(up)));
+}
+
+// Dims d .. d + 3 and d + half .. of head h of one row: rotated (q, k) and
+// written to q or through the block table to the pools.
+__device__ __forceinline__ void store_rope(const RowsArgs& a, int row, int h, int d, f32x4 lo,
+                                           f32x4 hi) {
+  const int half = a.hd / 2;
+  const int b = row / a.L;
+  const int l = row - b * a.L;
+  uint16_t o1[4], o2[4];
+  if (h < a.nq + a.nkv) {
+#pragma clang fp contract(off)
+    const float* cr = a.cos_t + static_cast<size_t>(l) * a.hd + d;
+    const float* sr = a.sin_t + static_cast<size_t>(l) * a.hd + d;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float x1 = bf2f(f2bf(lo[e]));
+      const float x2 = bf2f(f2bf(hi[e]));
+      const float a0 = x1 * cr[e];
+      const float b0 = -x2 * sr[e];
+      const float a1 = x2 * cr[half + e];
+      const float b1 = x1 * sr[half + e];
+      o1[e] = f2bf(a0 + b0);
+      o2[e] = f2bf(a1 + b1);
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      o1[e] = f2bf(lo[e]);
+      o2[e] = f2bf(hi[e]);
+    }
+  }
+  const u32x2 p1 = {o1[0] | static_cast<uint32_t>(o1[1]) << 16,
+                    o1[2] | static_cast<uint32_t>(o1[3]) << 16};
+  const u32x2 p2 = {o2[0] | static_cast<uint32_t>(o2[1]) << 16,
+                    o2[2] | static_cast<uint32_t>(o2[3]) << 16};
+  if (h < a.nq) {
+    uint16_t* qr = a.y + ((static_cast<size_t>(b) * a.nq + h) * a.L + l) * a.hd + d;
+    *reinterpret_cast<u32x2*>(qr) = p1;
+    *reinterpret_cast<u32x2*>(qr + half) = p2;
+    return;
+  }
+  const int pos = a.start + l;
+  const int page = pos >> a.pt_shift;
+  if (page >= a.max_pages) return;
+  const int slot = a.table[static_cast<size_t>(b) * a.max_pages + page];
+  if (static_cast<unsigned>(slot) >= static_cast<unsigned>(a.num_slots)) return;
+  const int off = pos & ((1 << a.pt_shift) - 1);
+  const bool is_k = h < a.nq + a.nkv;
+  const int kvh = is_k ? h - a.nq : h - a.nq - a.nkv;
+  const size_t head_page = static_cast<size_t>(slot) * a.nkv + kvh;
+  if (is_k) {
+    uint16_t* kr = a.k_pool + ((head_page << a.pt_shift) + off) * a.hd + d;
+    *reinterpret_cast<u32x2*>(kr) = p1;
+    *reinterpret_cast<u32x2*>(kr + half) = p2;
+  } else {
+    const int vb_shift = a.pt_shift < 5 ? a.pt_shift : 5;
+    const size_t blk = (head_page << (a.pt_shift - vb_shift)) + (off >> vb_shift);
+    const int col = off & ((1 << vb_shift) - 1);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      a.v_pool[((blk * a.hd + d + e) << vb_shift) + col] = o1[e];
+      a.v_pool[((blk * a.hd + d + half + e) << vb_shift) + col] = o2[e];
+    }
+  }
+}
+
+template <int CH, int MODE, int NW>
+__global__ __launch_bounds__(kWave* NW) void linear_rows_kernel(RowsArgs a) {
+  constexpr bool NORM = MODE != kPlain;
+  constexpr int T = MODE == kPlain ? 1 : 2;    // weight tiles of a wavefront
+  constexpr int SC = MODE == kPlain ? 12 : 6;  // k-steps of one register buffer
+  constexpr int LPR = kWave * NW / kRowsTile;  // lanes of one row
+  constexpr int CPL = kRowsUnit / 8 * CH / LPR;  // 16-byte chunks of one lane
+  // 16 bytes past whole 512-byte units: an odd multiple of 16 bytes between rows,
+  // so the 16 rows of a fragment lie on different LDS banks
+  constexpr int STRIDE = kRowsUnit * CH + 8;
+  __shared__ __align__(16) uint16_t lds[kRowsTile * STRIDE];
+  // workgroup i: XCD i % 8 takes column groups i % 8, i % 8 + 8, ...
+  const int xcd = blockIdx.x & 7;
+  const int idx = blockIdx.x >> 3;
+  const int group = uniform(xcd + 8 * (idx / a.row_groups));
+  const int row0 = uniform(kRowsTile * (idx % a.row_groups));
+  if (group >= a.groups) return;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = uniform(threadIdx.x / kWave);
+
+  // this lane's chunks of its row (a row past the end repeats the last one, a
+  // chunk past the row its last; neither is stored)
+  const int chunks = a.k / 8;
+  const int local = (kWave / LPR) * wave + lane / LPR;
+  const int c0 = lane % LPR;
+  const size_t at = static_cast<size_t>(min(row0 + local, a.rows - 1)) * a.k;
+  u32x4 v[CPL], d[NORM ? CPL : 1];
+  const uint16_t* dsrc = NORM && a.delta ? a.delta : a.x;
+#pragma unroll
+  for (int j = 0; j < CPL; ++j) {
+    const int c = min(c0 + LPR * j, chunks - 1);
+    v[j] = *reinterpret_cast<const u32x4*>(a.x + at + 8 * c);
+    if (NORM) d[j] = *reinterpret_cast<const u32x4*>(dsrc + at + 8 * c);
+  }
+
+  const int i16 = lane & 15;
+  const int kq = 8 * (lane >> 4);
+  const int steps = a.k / 32;
+  const int tile = uniform(NW * group + wave);
+  // wavefronts past the last tile read it again and store nothing
+  const int t = min(tile, a.tiles - 1);
+  int col[T];  // first column of each tile
+  int head = 0, dim = 0;
+  if (MODE == kPlain) {
+    col[0] = 16 * t;
+  } else if (MODE == kSwiglu) {
+    col[0] = 16 * t;
+    col[T - 1] = a.n + 16 * t;
+  } else {
+    const int per_head = a.hd / 32;
+    head = t / per_head;
+    dim = 16 * (t - head * per_head);
+    col[0] = head * a.hd + dim;
+    col[T - 1] = col[0] + a.hd / 2;
+  }
+  const uint16_t* wr[T];
+#pragma unroll
+  for (int j = 0; j < T; ++j) {
+    const int last = MODE == kRope ? col[j] + 15 : (j + 1) * a.n - 1;
+    wr[j] = a.w + static_cast<size_t>(min(col[j] + i16, last)) * a.k + kq;
+  }
+  auto load = [&](int s0, u32x4 (&wq)[T][SC]) {
+#pragma unroll
+    for (int i = 0; i < SC; ++i) {
+      const int s = min(s0 + i, steps - 1);
+#pragma unroll
+      for (int j = 0; j < T; ++j) wq[j][i] = *reinterpret_cast<const u32x4*>(wr[j] + 32 * s);
+    }
+  };
+  u32x4 wa[T][SC], wb[T][SC];
+  load(0, wa);
+  load(SC, wb);
+  asm volatile("" ::: "memory");  // the weights stay in flight under the norm
+
+  float inv = 1.f;
+  if (NORM) {
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < CPL; ++j) {
+      if (LPR * j >= chunks) continue;
+      const u32x4 sum = sum_chunks(v[j], d[NORM ? j : 0]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[j][e] = a.delta ? sum[e] : v[j][e];
+      if (c0 + LPR * j < chunks) ss = chunk_sumsq(v[j], ss);
+    }
+    inv = 1.f / sqrtf(group_sum<LPR>(ss) / static_cast<float>(a.k) + a.eps);
+  }
+  const bool writer = NORM && a.x_out != nullptr && group == 0 && row0 + local < a.rows;
+#pragma unroll
+  for (int j = 0; j < CPL; ++j) {
+    const int c = c0 + LPR * j;
+    if (c < chunks) {
+      if (writer) *reinterpret_cast<u32x4*>(a.x_out + at + 8 * c) = v[j];
+      if (NORM) v[j] = norm_chunk(v[j], *reinterpret_cast<const u32x4*>(a.ln + 8 * c), inv);
+      *reinterpret_cast<u32x4*>(lds + local * STRIDE + 8 * c) = v[j];
+    }
+  }
+  lds_barrier();
+
+  f32x4 acc[2][T];
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int j = 0; j < T; ++j) acc[m][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto product = [&](int s0, const u32x4 (&wq)[T][SC]) {
+#pragma unroll
+    for (int i = 0; i < SC; ++i) {
+      if (s0 + i < steps) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          const bf16x8 xr = *reinterpret_cast<const bf16x8*>(lds + (16 * m + i16) * STRIDE +
+                                                             32 * (s0 + i) + kq);
+#pragma unroll
+          for (int j = 0; j < T; ++j)
+            acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf16x8, wq[j][i]), xr, acc[m][j], 0, 0, 0);
+        }
+      }
+    }
+  };
+  for (int s0 = 0; s0 < steps; s0 += 2 * SC) {
+    product(s0, wa);
+    if (s0 + SC >= steps) break;
+    if (s0 + 2 * SC < steps) load(s0 + 2 * SC, wa);
+    product(s0 + SC, wb);
+    if (s0 + 3 * SC < steps) load(s0 + 3 * SC, wb);
+  }
+  if (tile >= a.tiles) return;
+  // lane (row i16 of its half): columns 4 (lane / 16) .. + 3 of the tile
+  const int sub = 4 * (lane >> 4);
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const int row = row0 + 16 * m + i16;
+    if (row >= a.rows) continue;
+    if (MODE == kRope) {
+      store_rope(a, row, head, dim + sub, acc[m][0], acc[m][T - 1]);
+    } else if (col[0] + sub < a.n) {
+      u32x2 o;
+      if (MODE == kSwiglu) {
+        uint16_t s[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] = swiglu_bf16(acc[m][0][e], acc[m][T - 1][e]);
+        o = u32x2{s[0] | static_cast<uint32_t>(s[1]) << 16,
+                  s[2] | static_cast<uint32_t>(s[3]) << 16};
+      } else {
+        o = u32x2{pack_bf16x2(acc[m][0][0], acc[m][0][1]),
+                  pack_bf16x2(acc[m][0][2], acc[m][0][3])};
+      }
+      *reinterpret_cast<u32x2*>(a.y + static_cast<size_t>(row) * a.n + col[0] + sub) = o;
+    }
+  }
+}
+
+template <int MODE>
+int launch_rows(const char* who, RowsArgs& a, hipStream_t stream) {
+  // The widest form prepares its rows half as often with eight wavefronts (3072
+  // columns: 18.1 us with four, 15.8 with eight); the narrow ones would leave most
+  // CUs idle (960 columns: 13.1 and 16.1 us; 576 columns, k 1536: 11.2 and 15.9).
+  constexpr int NW = MODE == kSwiglu ? 8 : 4;
+  a.groups = (a.tiles + NW - 1) / NW;
+  a.row_groups = (a.rows + kRowsTile - 1) / kRowsTile;
+  const long long grid = 8LL * ((a.groups + 7) / 8) * a.row_groups;
+  VOOM_REQUIRE(grid < (1LL << 31), "%s: too many rows", who);
+#define VOOM_ROWS(CH_)                                                                           \
+  case CH_:                                                                                      \
+    hipLaunchKernelGGL((linear_rows_kernel<CH_, MODE, NW>), dim3(static_cast<unsigned>(grid)), \
+                       dim3(kWave * NW), 0, stream, a);                                         \
+    break
+  switch ((a.k + kRowsUnit - 1) / kRowsUnit) {
+    VOOM_ROWS(1);
+    VOOM_ROWS(2);
+    VOOM_ROWS(3);
+    VOOM_ROWS(4);
+    VOOM_ROWS(5);
+    VOOM_ROWS(6);
+    VOOM_ROWS(7);
+    VOOM_ROWS(8);
+  }
+#undef VOOM_ROWS
+  return VOOM_LAUNCH_CHECK("linear_rows: kernel launch");
+}
+
 }  // namespace
 }  // namespace voom
 
@@ -658,6 +967,104 @@ extern "C" int voom_add_rms_norm_gemv(const void* x, const void* delta, const vo
   auto* xo = static_cast<uint16_t*>(x_out);
   return swiglu ? launch_gemv<true>(w, xv, dv, lw, eps, xo, yv, n, k, stream)
                 : launch_gemv<false>(w, xv, dv, lw, eps, xo, yv, n, k, stream);
+}
+
+namespace {
+int prepare_rows(const char* who, const void* x, const void* delta, const void* ln_weight,
+                 float eps, void* x_out, const void* weight, void* y, long long rows, int k,
+                 RowsArgs& a) {
+  VOOM_REQUIRE(weight && x && y, "%s: null pointer argument", who);
+  if (int rc = check_norm_prologue(who, x, delta, ln_weight, x_out)) return rc;
+  VOOM_REQUIRE(k > 0 && k % 32 == 0 && k <= 8 * kWave * 4,
+               "%s: k %d must be a positive multiple of 32 up to %d", who, k, 8 * kWave * 4);
+  VOOM_REQUIRE(rows > 0 && rows < (1LL << 24), "%s: bad row count", who);
+  VOOM_REQUIRE(reinterpret_cast<uintptr_t>(weight) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(y) % 16 == 0,
+               "%s: weight, x and the output must be 16-byte aligned", who);
+  a = RowsArgs{};
+  a.x = static_cast<const uint16_t*>(x);
+  a.delta = static_cast<const uint16_t*>(delta);
+  a.ln = static_cast<const uint16_t*>(ln_weight);
+  a.x_out = static_cast<uint16_t*>(x_out);
+  a.w = static_cast<const uint16_t*>(weight);
+  a.y = static_cast<uint16_t*>(y);
+  a.rows = static_cast<int>(rows);
+  a.k = k;
+  a.eps = eps;
+  return VOOM_OK;
+}
+}  // namespace
+
+extern "C" int voom_linear_rows(const void* x, const void* weight, void* y, int rows, int n, int k,
+                                hipStream_t stream) {
+  const char* who = "linear_rows";
+  RowsArgs a;
+  if (int rc = prepare_rows(who, x, nullptr, nullptr, 0.f, nullptr, weight, y, rows, k, a))
+    return rc;
+  VOOM_REQUIRE(n > 0 && n % 8 == 0 && n < (1 << 28), "%s: n %d must be a positive multiple of 8",
+               who, n);
+  a.n = n;
+  a.tiles = (n + 15) / 16;
+  return launch_rows<kPlain>(who, a, stream);
+}
+
+extern "C" int voom_norm_swiglu_rows(const void* x, const void* delta, const void* ln_weight,
+                                     float eps, void* x_out, const void* weight, void* y, int rows,
+                                     int n, int k, hipStream_t stream) {
+  const char* who = "norm_swiglu_rows";
+  RowsArgs a;
+  VOOM_REQUIRE(ln_weight != nullptr, "%s: null pointer argument", who);
+  if (int rc = prepare_rows(who, x, delta, ln_weight, eps, x_out, weight, y, rows, k, a)) return rc;
+  VOOM_REQUIRE(n > 0 && n % 8 == 0 && n < (1 << 28), "%s: n %d must be a positive multiple of 8",
+               who, n);
+  a.n = n;
+  a.tiles = (n + 15) / 16;
+  return launch_rows<kSwiglu>(who, a, stream);
+}
+
+extern "C" int voom_qkv_rope_append_rows(const void* w_qkv, const void* x, const void* delta,
+                                         const void* ln_weight, float eps, void* x_out,
+                                         const float* cos_table, const float* sin_table, void* q,
+                                         void* k_pool, void* v_pool, const int32_t* block_table,
+                                         int batch, int seq, int start, int num_q_heads,
+                                         int num_kv_heads, int head_dim, int k, int page_tokens,
+                                         int max_pages, int num_slots, hipStream_t stream) {
+  const char* who = "qkv_rope_append_rows";
+  RowsArgs a;
+  VOOM_REQUIRE(ln_weight && cos_table && sin_table && k_pool && v_pool && block_table,
+               "%s: null pointer argument", who);
+  VOOM_REQUIRE(batch > 0 && seq > 0, "%s: bad geometry", who);
+  if (int rc = prepare_rows(who, x, delta, ln_weight, eps, x_out, w_qkv, q,
+                            static_cast<long long>(batch) * seq, k, a))
+    return rc;
+  VOOM_REQUIRE(num_q_heads > 0 && num_kv_heads > 0 && num_q_heads < (1 << 14) &&
+                   num_kv_heads < (1 << 14) && head_dim > 0 && head_dim <= 1024 &&
+                   head_dim % 32 == 0,
+               "%s: bad head geometry (head_dim a multiple of 32)", who);
+  VOOM_REQUIRE(is_pow2(page_tokens) && page_tokens <= 4096 && max_pages > 0 && num_slots > 0,
+               "%s: bad page geometry", who);
+  VOOM_REQUIRE(start >= 0 && static_cast<long long>(start) + seq < (1LL << 31),
+               "%s: bad start %d", who, start);
+  VOOM_REQUIRE(reinterpret_cast<uintptr_t>(k_pool) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(v_pool) % 16 == 0,
+               "%s: pools must be 16-byte aligned", who);
+  a.n = (num_q_heads + 2 * num_kv_heads) * head_dim;
+  a.tiles = (num_q_heads + 2 * num_kv_heads) * (head_dim / 32);
+  a.cos_t = cos_table;
+  a.sin_t = sin_table;
+  a.k_pool = static_cast<uint16_t*>(k_pool);
+  a.v_pool = static_cast<uint16_t*>(v_pool);
+  a.table = block_table;
+  a.L = seq;
+  a.start = start;
+  a.nq = num_q_heads;
+  a.nkv = num_kv_heads;
+  a.hd = head_dim;
+  a.pt_shift = ilog2(page_tokens);
+  a.max_pages = max_pages;
+  a.num_slots = num_slots;
+  return launch_rows<kRope>(who, a, stream);
 }
 
 extern "C" int voom_lm_head_argmax(const void* x, const void* delta, const void* ln_weight,

@@ -14,10 +14,12 @@ drive the cache:
     (runtime/engine.py:8459-8503): embed the pending token, sweep the
     layers at ``kv.offset``, final norm + tied lm_head, argmax.
 
-GEMMs are PyTorch-ROCm (hipBLASLt); the residual add + RMSNorm, RoPE with
-the q/k/v split, and SwiGLU are fused HIP kernels (voom_add_rms_norm,
-voom_rope_split, voom_silu_mul), and every attention call is the paged HIP
-kernel.  ``generate_graph`` replays each decode step from one captured HIP
+A prompt's projections carry the residual add + RMSNorm, RoPE with the page
+write, and SwiGLU in their own launches (voom_qkv_rope_append_rows,
+voom_norm_swiglu_rows, voom_linear_rows).  Where the products outweigh the
+launches they are PyTorch-ROCm GEMMs (hipBLASLt) between the separate kernels
+(voom_add_rms_norm, voom_rope_split, voom_silu_mul).  Every attention call is
+the paged HIP kernel.  ``generate_graph`` replays each decode step from one captured HIP
 graph.  Weights use the Hugging Face Llama parameter names so that an
 in-code ``LlamaForCausalLM`` can load them.
 """
@@ -85,6 +87,16 @@ def random_weights(cfg: DecoderConfig, seed: int = 0, device=None,
     if device is not None:
         w = {k: v.to(device) for k, v in w.items()}
     return w
+
+
+# A prompt's layers take the fused row projections up to this many multiply-adds
+# (rows x the layer's weights), where five launches beat the library products and
+# the launches around them, beyond it the products' rate decides: hidden 576,
+# 30 layers, 1536 rows (5.4e9) 4.0 against 6.1 ms and 4096 rows (1.4e10) 9.4
+# against 7.1; hidden 2048, 8 layers, 256 rows (6.4e9) 1.1 against 1.5 ms and 512
+# rows (1.3e10) 1.9 against 1.6; hidden 256, 8 layers, 8192 rows (6.4e9) 2.3
+# against 2.5 ms.
+FUSED_MAX_WORK = 6 << 30
 
 
 class PagedDecoder:
@@ -172,6 +184,37 @@ class PagedDecoder:
                        x_out=spare)
         return ops.gemv(act, lw["down"]), spare, x
 
+    def _rows_fused(self, x: torch.Tensor) -> bool:
+        """Whether ``_block_rows`` takes the rows of x: shapes that its kernels
+        hold, and more than the one row of the GEMV kernels."""
+        cfg = self.cfg
+        H, inter = cfg.hidden_size, cfg.intermediate_size
+        qd, kvd = cfg.num_attention_heads * cfg.head_dim, cfg.num_key_value_heads * cfg.head_dim
+        rows = x.shape[0] * x.shape[1]
+        return (rows > 1 and rows * H * (2 * qd + 2 * kvd + 3 * inter) <= FUSED_MAX_WORK
+                and cfg.head_dim % 32 == 0 and H % 32 == 0 and inter % 32 == 0
+                and max(H, inter, qd) <= ops.GEMV_MAX_K)
+
+    def _block_rows(self, x: torch.Tensor, spare: torch.Tensor, delta: torch.Tensor | None,
+                    layer: int, kv: PagedKVCache, cos: torch.Tensor, sin: torch.Tensor):
+        """``_block`` for the rows of a prompt in five launches: residual adds,
+        RMSNorms, RoPE, the page write and SwiGLU are folded into the projections.
+        Streams and returns as in ``_block_token``."""
+        cfg = self.cfg
+        lw = self.layers[layer]
+        B, L, _ = x.shape
+        nq, nkv, hd, eps = (cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim,
+                            cfg.rms_norm_eps)
+        q = kv.project_append(layer, x, lw["qkv"], cos, sin, nq, nkv, ln_weight=lw["ln1"], eps=eps,
+                              delta=delta, x_out=None if delta is None else spare)
+        if delta is not None:
+            x, spare = spare, x
+        attn = (kv.attend(layer, q, scale=hd ** -0.5) if L == 1
+                else kv.attend_prefill(layer, q, scale=hd ** -0.5))
+        o = ops.linear_rows(attn.transpose(1, 2).reshape(B, L, nq * hd), lw["o"])
+        act = ops.norm_swiglu_rows(x, lw["gate_up"], lw["ln2"], eps, delta=o, x_out=spare)
+        return ops.linear_rows(act, lw["down"]), spare, x
+
     def _block(self, x: torch.Tensor, delta: torch.Tensor | None, layer: int,
                kv: PagedKVCache, cos: torch.Tensor, sin: torch.Tensor,
                graph: bool = False) -> torch.Tensor:
@@ -212,11 +255,18 @@ class PagedDecoder:
         cos, sin = self._rope_tables(torch.arange(offset, offset + L, device=self.device))
         x = self.embed[tokens]
         delta = None
-        for layer in range(self.cfg.num_hidden_layers):
-            delta = self._block(x, delta, layer, kv, cos, sin)
+        fused = self._rows_fused(x)
+        spare = torch.empty_like(x) if fused else None
+        for layer, lw in enumerate(self.layers):
+            if fused and (lw["o"].data_ptr() | lw["down"].data_ptr() | lw["qkv"].data_ptr()
+                          | lw["gate_up"].data_ptr()) % 16 == 0:
+                delta, x, spare = self._block_rows(x, spare, delta, layer, kv, cos, sin)
+            else:
+                delta = self._block(x, delta, layer, kv, cos, sin)
+        if last_only:  # the rows before the last one end here
+            x = x[:, -1:].contiguous()
+            delta = None if delta is None else delta[:, -1:].contiguous()
         x = self._norm(x, self.final_norm, delta)
-        if last_only:
-            x = x[:, -1:]
         return self._linear(x, self.embed).float()
 
     # ---- one decode step in a HIP graph ------------------------------------------

@@ -780,11 +780,30 @@ class PagedKVCache:
         if v.shape != k.shape:
             raise ValueError("k and v shapes differ")
 
-        def write(pool, pos):
+        def write(pool, start):
             ops.append_kv(k.contiguous(), v.contiguous(), pool.k, pool.v, self._tables[layer],
-                          pos)
+                          self._positions(start))
 
         self._append(layer, k.shape[2], write)
+
+    def project_append(self, layer: int, h: torch.Tensor, w_qkv: torch.Tensor,
+                       cos: torch.Tensor, sin: torch.Tensor, num_q_heads: int,
+                       num_kv_heads: int, **norm) -> torch.Tensor:
+        """``append`` with the fused qkv projection of h [B, L, K] and its RoPE
+        folded in, one launch; returns q [B, NQ, L, D].  ``norm`` (ln_weight, eps,
+        delta, x_out) is the residual add + RMSNorm of h in front."""
+        D = cos.shape[-1]
+        self._set_geometry(("kv", h.shape[0], num_kv_heads, D), h.dtype)
+        q = None
+
+        def write(pool, start):
+            nonlocal q
+            q = ops.qkv_rope_append_rows(h, w_qkv, cos, sin, pool.k, pool.v,
+                                         self._tables[layer], start, num_q_heads, num_kv_heads, D,
+                                         **norm)
+
+        self._append(layer, h.shape[1], write)
+        return q
 
     def append_latent(self, layer: int, lat: torch.Tensor) -> None:
         """Write latent rows lat [B, L, latent_dim] ([c_kv | k_rope]) after the
@@ -792,10 +811,14 @@ class PagedKVCache:
         (runtime/kv_cache.py:99-105) as a slot write into the latent pool."""
         self._init_latent(lat)
 
-        def write(pool, pos):
-            ops.append_rows(lat.contiguous(), pool.lat, self._tables[layer], pos)
+        def write(pool, start):
+            ops.append_rows(lat.contiguous(), pool.lat, self._tables[layer],
+                            self._positions(start))
 
         self._append(layer, lat.shape[1], write)
+
+    def _positions(self, start: int) -> torch.Tensor:
+        return torch.full((self._batch,), start, dtype=torch.int32, device=self.device)
 
     def _append(self, layer: int, L: int, write) -> None:
         B = self._batch
@@ -813,7 +836,7 @@ class PagedKVCache:
                 self._open_slots[layer][page] = cols[page]
             self._set_table_cols(layer, cols)
         if L:
-            write(pool, torch.full((B,), start, dtype=torch.int32, device=self.device))
+            write(pool, start)
         self._len[layer] = end
         pages = self._pages[layer]
         while (len(pages) + 1) * PT <= end:

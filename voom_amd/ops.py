@@ -858,6 +858,69 @@ def qkv_rope_append(x: torch.Tensor, w_qkv: torch.Tensor, cos: torch.Tensor, sin
     return q
 
 
+def linear_rows(x: torch.Tensor, weight: torch.Tensor, *,
+                stream: torch.cuda.Stream | None = None) -> torch.Tensor:
+    """``gemv`` for any number of rows: x [..., K] . weight^T -> [..., N]."""
+    dev = _require_device(x, weight)
+    _require(x.dtype == weight.dtype == torch.bfloat16, "bf16 x and weight")
+    _require(weight.dim() == 2 and x.shape[-1] == weight.shape[1], "weight [N, K] with K = x's")
+    n, K = weight.shape
+    y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=dev)
+    _lib.call("voom_linear_rows", _ptr(x), _ptr(weight), _ptr(y), x.numel() // max(K, 1), n, K,
+              _stream(stream))
+    return y
+
+
+def norm_swiglu_rows(x: torch.Tensor, weight: torch.Tensor, ln_weight: torch.Tensor, eps: float,
+                     *, delta: torch.Tensor | None = None, x_out: torch.Tensor | None = None,
+                     stream: torch.cuda.Stream | None = None) -> torch.Tensor:
+    """``gemv(swiglu=True, ln_weight=...)`` for any number of rows: x [..., K] and the
+    fused [gate; up] weight [2I, K] -> [..., I]."""
+    dev = _require_device(x, weight, ln_weight, delta, x_out)
+    _require(x.dtype == weight.dtype == torch.bfloat16, "bf16 x and weight")
+    _norm_prologue(x, ln_weight, delta, x_out)
+    _require(weight.dim() == 2 and x.shape[-1] == weight.shape[1] and weight.shape[0] % 2 == 0,
+             "weight [2I, K] with K = x's")
+    n, K = weight.shape[0] // 2, weight.shape[1]
+    y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=dev)
+    _lib.call("voom_norm_swiglu_rows", _ptr(x), _ptr(delta), _ptr(ln_weight), float(eps),
+              _ptr(x_out), _ptr(weight), _ptr(y), x.numel() // max(K, 1), n, K, _stream(stream))
+    return y
+
+
+def qkv_rope_append_rows(x: torch.Tensor, w_qkv: torch.Tensor, cos: torch.Tensor,
+                         sin: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
+                         block_table: torch.Tensor, start: int, num_q_heads: int,
+                         num_kv_heads: int, head_dim: int, *, ln_weight: torch.Tensor,
+                         eps: float, delta: torch.Tensor | None = None, x_out: torch.Tensor | None = None,
+                         stream: torch.cuda.Stream | None = None) -> torch.Tensor:
+    """x [B, L, K] through the residual add + RMSNorm of ``gemv``'s prologue, the
+    fused qkv projection, RoPE with cos/sin [L, hd] fp32 and the page write of k
+    and v at positions start .. start + L - 1, one launch; returns q [B, nq, L, hd]."""
+    dev = _require_device(x, w_qkv, cos, sin, k_pool, v_pool, block_table, ln_weight, delta,
+                          x_out)
+    _norm_prologue(x, ln_weight, delta, x_out)
+    nq, nkv, hd = int(num_q_heads), int(num_kv_heads), int(head_dim)
+    _require(x.dim() == 3 and w_qkv.dim() == 2 and x.shape[-1] == w_qkv.shape[1],
+             "x [B, L, K] and w_qkv [N, K]")
+    B, L, K = x.shape
+    _require(w_qkv.shape[0] == (nq + 2 * nkv) * hd, "w_qkv rows must be (nq + 2 nkv) * hd")
+    _require(x.dtype == w_qkv.dtype == k_pool.dtype == v_pool.dtype == torch.bfloat16, "bf16")
+    _require(cos.dtype == sin.dtype == torch.float32
+             and tuple(cos.shape) == (L, hd) == tuple(sin.shape), "fp32 [L, hd] tables")
+    slots, NKVp, PT, Dp = k_pool.shape
+    _require(NKVp == nkv and Dp == hd, "pool geometry does not match the heads")
+    _check_v_pool(v_pool, slots, nkv, hd, PT)
+    _require(block_table.dtype == torch.int32 and block_table.dim() == 2
+             and block_table.shape[0] == B, "block_table must be int32 [B, max_pages]")
+    q = torch.empty((B, nq, L, hd), dtype=x.dtype, device=dev)
+    _lib.call("voom_qkv_rope_append_rows", _ptr(w_qkv), _ptr(x), _ptr(delta), _ptr(ln_weight),
+              float(eps), _ptr(x_out), _ptr(cos), _ptr(sin), _ptr(q), _ptr(k_pool), _ptr(v_pool),
+              _ptr(block_table), B, L, int(start), nq, nkv, hd, K, PT, block_table.shape[1], slots,
+              _stream(stream))
+    return q
+
+
 def split_kv_b(kv_b: torch.Tensor, num_heads: int, dn: int, dv: int):
     """kv_b_proj weight [H*(dn+dv), C] -> (W_UK [H, dn, C], W_UV^T [H, C, dv]), contiguous.
 
