@@ -10,7 +10,6 @@ import os
 import shutil
 import subprocess
 import sys
-import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
@@ -21,8 +20,6 @@ LIB_NAME = "libvoom_hip.so"
 LIB_PATH = PKG_DIR / LIB_NAME
 # bench-only probe kernels (csrc/bench), linked against LIB_NAME
 CALIB_LIB_PATH = PKG_DIR / "libvoom_calibrate.so"
-# the Python bindings of LIB_NAME's C ABI (csrc/host)
-CALLS_PATH = PKG_DIR / f"_calls{sysconfig.get_config_var('EXT_SUFFIX')}"
 ARCH = "gfx950"
 
 # Packed-fp32 instructions are disabled for every device pass (the flag is
@@ -57,35 +54,16 @@ def _run(cmd: list[str]) -> str:
     return err
 
 
-def _link(cc: str, objs: list[Path], out: Path, extra: list[str], flags=HIP_FLAGS) -> str:
+def _link(cc: str, objs: list[Path], out: Path, extra: list[str]) -> str:
     tmp = out.with_suffix(".so.tmp")
-    err = _run([cc, *flags, "-shared", "-o", str(tmp), *map(str, objs), *extra])
+    err = _run([cc, *HIP_FLAGS, "-shared", "-o", str(tmp), *map(str, objs), *extra])
     os.replace(tmp, out)
     return err
 
 
-def _calls_commands(obj: Path) -> tuple[list[str], list[str]]:
-    """The compile command of the Python bindings and their link's extra flags."""
-    import torch
-
-    inc = Path(torch.__file__).parent / "include"
-    cxx = os.environ.get("CXX") or "g++"
-    rocm = Path(hipcc()).parent.parent / "include"
-    compile_cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__",
-                   f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-                   f"-I{sysconfig.get_paths()['include']}", f"-I{inc}",
-                   f"-I{inc / 'torch' / 'csrc' / 'api' / 'include'}", f"-I{rocm}",
-                   "-c", "-o", str(obj), str(CSRC / "host" / "calls.cpp")]
-    # torch's libraries are loaded before the bindings; its folder is not recorded
-    link = [f"-L{PKG_DIR}", "-lvoom_hip", f"-L{inc.parent / 'lib'}", "-ltorch_python",
-            "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN"]
-    return compile_cmd, link
-
-
 def build(verbose: bool = False) -> Path:
     """Compile every kernel source into one shared library and return its path;
-    the bench-only probes (csrc/bench) go into libvoom_calibrate.so beside it, the
-    Python bindings (csrc/host) into the module ``_calls``.
+    the bench-only probes (csrc/bench) go into libvoom_calibrate.so beside it.
 
     Each source is compiled to an object in its own hipcc process (in
     parallel; every translation unit holds its kernels and their launchers,
@@ -98,9 +76,6 @@ def build(verbose: bool = False) -> Path:
     with tempfile.TemporaryDirectory(prefix="voom_build_") as tdir:
         objs = [Path(tdir) / f"{i}_{src.name}.o" for i, src in enumerate(every)]
         cmds = [[cc, *HIP_FLAGS, "-c", "-o", str(obj), str(src)] for src, obj in zip(every, objs)]
-        calls_obj = Path(tdir) / "calls.o"
-        calls_cmd, calls_link = _calls_commands(calls_obj)
-        cmds.append(calls_cmd)
         if verbose:
             for cmd in cmds:
                 print(" ".join(cmd), flush=True)
@@ -109,7 +84,6 @@ def build(verbose: bool = False) -> Path:
         errs.append(_link(cc, objs[:len(srcs)], LIB_PATH, []))
         errs.append(_link(cc, objs[len(srcs):], CALIB_LIB_PATH,
                           [f"-L{PKG_DIR}", "-lvoom_hip", "-Wl,-rpath,$ORIGIN"]))
-        errs.append(_link(calls_cmd[0], [calls_obj], CALLS_PATH, calls_link, flags=[]))
     if verbose:
         for err in errs:
             if err.strip():

@@ -1,5 +1,4 @@
-"""Bindings of libvoom_hip.so (the C ABI declared in include/voom_hip.h): compiled
-ones for the operations (``call``, ``calls``), ctypes for everything else.
+"""ctypes binding of libvoom_hip.so (the C ABI declared in include/voom_hip.h).
 
 There is no fallback: if the library is missing or does not load, every
 operation raises.  Return codes map to exceptions the way the reference's
@@ -14,13 +13,12 @@ import ctypes
 import threading
 from ctypes import c_float, c_int, c_longlong, c_size_t, c_void_p
 
-from ._build import CALLS_PATH, LIB_PATH
+from ._build import LIB_PATH
 
 VOOM_EINVAL = -1
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
-_calls = None
 
 _P = c_void_p
 # name -> (restype, argtypes)
@@ -115,7 +113,7 @@ class VoomLibraryError(RuntimeError):
 
 def lib() -> ctypes.CDLL:
     """Load (once) and return the HIP library; raise if it is unavailable."""
-    global _lib, _calls
+    global _lib
     if _lib is not None:
         return _lib
     with _lock:
@@ -125,16 +123,12 @@ def lib() -> ctypes.CDLL:
                     f"{LIB_PATH} is not built; run __graft_entry__.build() first")
             try:
                 handle = ctypes.CDLL(str(LIB_PATH))
-                import torch  # noqa: F401  (the bindings link against its libraries)
-
-                from . import _calls as bindings
-            except (OSError, ImportError) as exc:  # pragma: no cover - depends on the box
-                raise VoomLibraryError(f"cannot load {LIB_PATH} or {CALLS_PATH}: {exc}") from exc
+            except OSError as exc:  # pragma: no cover - depends on the box
+                raise VoomLibraryError(f"cannot load {LIB_PATH}: {exc}") from exc
             for name, (res, args) in SIGNATURES.items():
                 fn = getattr(handle, name)
                 fn.restype = res
                 fn.argtypes = args
-            _calls = bindings
             _lib = handle
             atexit.register(_teardown)
     return _lib
@@ -183,20 +177,5 @@ def check(rc: int, what: str) -> None:
     raise RuntimeError(f"{what}: HIP error {rc}: {msg}")
 
 
-def calls():
-    """The compiled bindings of the C ABI (csrc/host/calls.cpp)."""
-    if _calls is None:
-        lib()
-    return _calls
-
-
 def call(name: str, *args) -> None:
-    """One entry point through the compiled bindings: pointers as tensors, integers
-    or None; other forms (ctypes objects), which they refuse before the call, through
-    ctypes."""
-    try:
-        rc = getattr(_calls or calls(), name)(*args)
-    except TypeError:
-        rc = getattr(lib(), name)(*(a.data_ptr() if hasattr(a, "data_ptr") else a for a in args))
-    if rc:
-        check(rc, name)
+    check(getattr(lib(), name)(*args), name)

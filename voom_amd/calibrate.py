@@ -16,7 +16,7 @@ import torch
 
 from . import _lib
 from ._build import CALIB_LIB_PATH
-from .ops import _require, _require_device, _stream
+from .ops import _ptr, _require, _require_device, _stream
 
 _P = c_void_p
 SIGNATURES: dict[str, tuple[object, list[object]]] = {
@@ -46,10 +46,6 @@ def lib() -> CDLL:
                     fn.argtypes = args
                 _handle = h
     return _handle
-
-
-def _ptr(t: torch.Tensor | None) -> int | None:
-    return None if t is None else int(t.data_ptr())
 
 
 def _call(name: str, *args) -> None:

@@ -39,14 +39,26 @@ def _stream(stream: torch.cuda.Stream | None) -> int:
     return int(torch.cuda.current_stream().cuda_stream)
 
 
+def _ptr(t: torch.Tensor | None) -> int | None:
+    return None if t is None else int(t.data_ptr())
+
+
 def _require(cond: bool, msg: str) -> None:
     if not cond:
         raise ValueError(msg)
 
 
-def _require_device(*tensors: torch.Tensor | None) -> torch.device:
-    """The one device of the given contiguous tensors (None skipped)."""
-    return _lib.calls().require_device(*tensors)
+def _require_device(*tensors: torch.Tensor) -> torch.device:
+    dev = None
+    for t in tensors:
+        if t is None:
+            continue
+        _require(t.is_cuda, "voom_amd ops need ROCm device tensors (no CPU fallback exists)")
+        _require(t.is_contiguous(), "voom_amd ops need contiguous tensors")
+        if dev is None:
+            dev = t.device
+        _require(t.device == dev, "all tensors must be on the same device")
+    return dev
 
 
 def _side_stream(stream: torch.cuda.Stream | None) -> torch.cuda.Stream | None:
@@ -108,7 +120,7 @@ def check_block_table(block_table: torch.Tensor, ctx_lens: torch.Tensor, num_slo
         raise RuntimeError("bounds checks synchronise and cannot run under graph capture")
     B, max_pages = block_table.shape
     status = torch.zeros(4, dtype=torch.int32, device=block_table.device)
-    _lib.call("voom_check_block_table", block_table, ctx_lens, status, B,
+    _lib.call("voom_check_block_table", _ptr(block_table), _ptr(ctx_lens), _ptr(status), B,
               max_pages, int(page_tokens), int(num_slots), _stream(stream))
     bad = status.cpu().tolist()
     if bad[1]:
@@ -129,8 +141,8 @@ def check_selection(sel: torch.Tensor, sel_lens: torch.Tensor, block_table: torc
     B, k = sel.shape
     max_pages = block_table.shape[1]
     status = torch.zeros(4, dtype=torch.int32, device=sel.device)
-    _lib.call("voom_check_selection", sel, sel_lens, block_table,
-              status, B, k, max_pages, int(page_tokens), int(num_slots), _stream(stream))
+    _lib.call("voom_check_selection", _ptr(sel), _ptr(sel_lens), _ptr(block_table),
+              _ptr(status), B, k, max_pages, int(page_tokens), int(num_slots), _stream(stream))
     bad = status.cpu().tolist()
     if bad[3]:
         raise ValueError(f"{bad[3]} selection counts lie outside [0, {k}]")
@@ -151,8 +163,8 @@ def check_position_free_pages(block_table: torch.Tensor, key_positions: torch.Te
     if TK == 0:
         return
     status = torch.zeros(4, dtype=torch.int32, device=key_positions.device)
-    _lib.call("voom_check_position_free_pages", block_table, key_positions,
-              status, TK, int(block_size), int(num_pages), int(max_position), _stream(stream))
+    _lib.call("voom_check_position_free_pages", _ptr(block_table), _ptr(key_positions),
+              _ptr(status), TK, int(block_size), int(num_pages), int(max_position), _stream(stream))
     bad = status.cpu().tolist()
     if bad[0]:
         raise ValueError(f"block table holds {bad[0]} page ids outside [0, {num_pages})")
@@ -166,8 +178,8 @@ def default_splits() -> int:
 
 def gqa_workspace_bytes(batch: int, num_q_heads: int, num_kv_heads: int, head_dim: int,
                         num_splits: int) -> int:
-    return int(_lib.calls().voom_paged_gqa_workspace_bytes(batch, num_q_heads, num_kv_heads,
-                                                           head_dim, num_splits))
+    return int(_lib.lib().voom_paged_gqa_workspace_bytes(batch, num_q_heads, num_kv_heads,
+                                                        head_dim, num_splits))
 
 
 def _check_v_pool(v_pool, slots, NKV, D, PT):
@@ -232,8 +244,8 @@ def paged_gqa_decode(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor
     if out is None:
         out = torch.empty((B, NQ, D), dtype=torch.bfloat16, device=q.device)
     lse = torch.empty((B, NQ), dtype=torch.float32, device=q.device) if return_lse else None
-    _lib.call("voom_paged_gqa_decode", q, k_pool, v_pool, block_table,
-              ctx_lens, out, lse, ws, need, B, NQ, NKV, D, PT,
+    _lib.call("voom_paged_gqa_decode", _ptr(q), _ptr(k_pool), _ptr(v_pool), _ptr(block_table),
+              _ptr(ctx_lens), _ptr(out), _ptr(lse), _ptr(ws), need, B, NQ, NKV, D, PT,
               max_pages, slots, scale, num_splits, _stream(stream))
     out = out.reshape(q_shape)
     return (out, lse) if return_lse else out
@@ -249,8 +261,8 @@ def paged_gqa_partials(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tens
     using the same geometry, num_splits and workspace."""
     q, (B, NQ, NKV, D, PT, max_pages, slots), scale, num_splits, ws, need = _gqa_plan(
         q, k_pool, v_pool, block_table, ctx_lens, None, scale, num_splits, ws)
-    _lib.call("voom_paged_gqa_partials", q, k_pool, v_pool,
-              block_table, ctx_lens, ws, need, B, NQ, NKV, D, PT, max_pages,
+    _lib.call("voom_paged_gqa_partials", _ptr(q), _ptr(k_pool), _ptr(v_pool),
+              _ptr(block_table), _ptr(ctx_lens), _ptr(ws), need, B, NQ, NKV, D, PT, max_pages,
               slots, scale, num_splits, _stream(stream))
     return ws
 
@@ -265,7 +277,7 @@ def paged_gqa_combine(ctx_lens: torch.Tensor, out: torch.Tensor, ws: torch.Tenso
     B, NQ, D = out.shape
     need = gqa_workspace_bytes(B, NQ, num_kv_heads, D, num_splits)
     _require(ws.numel() * ws.element_size() >= need, "workspace too small")
-    _lib.call("voom_paged_gqa_combine", ctx_lens, out, lse, ws, need, B,
+    _lib.call("voom_paged_gqa_combine", _ptr(ctx_lens), _ptr(out), _ptr(lse), _ptr(ws), need, B,
               NQ, num_kv_heads, D, page_tokens, max_pages, num_splits, _stream(stream))
     return out
 
@@ -297,10 +309,10 @@ def paged_gqa_prefill(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tenso
     out = torch.empty((B, L, NQ, D), dtype=torch.bfloat16, device=dev)
     # key-split partials: allocated per call, so calls on several streams or
     # threads never share them
-    need = int(_lib.calls().voom_paged_gqa_prefill_workspace_bytes(B, NQ, NKV, D, L, seq_len))
+    need = int(_lib.lib().voom_paged_gqa_prefill_workspace_bytes(B, NQ, NKV, D, L, seq_len))
     ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
-    _lib.call("voom_paged_gqa_prefill", q, k_pool, v_pool, block_table,
-              out, ws, need, B, NQ, NKV, D, PT, block_table.shape[1], slots, L,
+    _lib.call("voom_paged_gqa_prefill", _ptr(q), _ptr(k_pool), _ptr(v_pool), _ptr(block_table),
+              _ptr(out), _ptr(ws), need, B, NQ, NKV, D, PT, block_table.shape[1], slots, L,
               int(seq_len), float(D ** -0.5 if scale is None else scale), _stream(None))
     return out
 
@@ -317,8 +329,8 @@ def merge_attn_states(o_a: torch.Tensor, lse_a: torch.Tensor, o_b: torch.Tensor,
     _require(lse_a.dtype == lse_b.dtype == torch.float32, "lse must be float32")
     out = torch.empty_like(o_a)
     lse = torch.empty(lse_a.shape, dtype=torch.float32, device=dev)
-    _lib.call("voom_merge_attn_states", o_a, lse_a, o_b, lse_b,
-              out, lse, rows, D, _stream(stream))
+    _lib.call("voom_merge_attn_states", _ptr(o_a), _ptr(lse_a), _ptr(o_b), _ptr(lse_b),
+              _ptr(out), _ptr(lse), rows, D, _stream(stream))
     return out, lse
 
 
@@ -340,7 +352,7 @@ def fold_attn_state(o_acc: torch.Tensor, lse_acc: torch.Tensor, o_b: torch.Tenso
     D = o_b.shape[-1]
     rows = o_b.numel() // D
     _require(lse_acc.numel() == rows == lse_b.numel(), "lse must have one entry per row")
-    _lib.call("voom_fold_attn_state", o_acc, lse_acc, o_b, lse_b,
+    _lib.call("voom_fold_attn_state", _ptr(o_acc), _ptr(lse_acc), _ptr(o_b), _ptr(lse_b),
               rows, D, int(bool(init)), _stream(stream))
 
 
@@ -360,8 +372,8 @@ def append_kv(k_new: torch.Tensor, v_new: torch.Tensor, k_pool: torch.Tensor,
              "block_table and positions must be int32")
     _require(block_table.shape[0] == B and tuple(positions.shape) == (B,),
              "block_table/positions batch mismatch")
-    _lib.call("voom_append_kv", k_new, v_new, k_pool, v_pool,
-              block_table, positions, B, NKV, L, D, PT, block_table.shape[1],
+    _lib.call("voom_append_kv", _ptr(k_new), _ptr(v_new), _ptr(k_pool), _ptr(v_pool),
+              _ptr(block_table), _ptr(positions), B, NKV, L, D, PT, block_table.shape[1],
               slots, _stream(stream))
 
 
@@ -375,7 +387,7 @@ def gather_kv(k_pool: torch.Tensor, v_pool: torch.Tensor, block_table: torch.Ten
     _require(block_table.dtype == torch.int32, "block_table must be int32")
     k = torch.empty((B, NKV, seq_len, D), dtype=k_pool.dtype, device=dev)
     v = torch.empty_like(k)
-    _lib.call("voom_gather_kv", k_pool, v_pool, block_table, k, v,
+    _lib.call("voom_gather_kv", _ptr(k_pool), _ptr(v_pool), _ptr(block_table), _ptr(k), _ptr(v),
               B, NKV, seq_len, D, PT, block_table.shape[1], slots, _stream(stream))
     return k, v
 
@@ -396,7 +408,7 @@ def byteplane_split(src: torch.Tensor, lo: torch.Tensor | None = None,
     hi = torch.empty(n, dtype=torch.uint8, device=dev) if hi is None else hi
     _require(lo.numel() >= n and hi.numel() >= n and lo.dtype == hi.dtype == torch.uint8,
              "planes must be uint8 with >= numel bytes")
-    _lib.call("voom_byteplane_split", src, lo, hi, n, _stream(stream))
+    _lib.call("voom_byteplane_split", _ptr(src), _ptr(lo), _ptr(hi), n, _stream(stream))
     return lo, hi
 
 
@@ -408,7 +420,7 @@ def byteplane_merge(lo: torch.Tensor, hi: torch.Tensor, out: torch.Tensor, *,
     n = out.numel()
     _require(lo.numel() >= n and hi.numel() >= n and lo.dtype == hi.dtype == torch.uint8,
              "planes must be uint8 with >= numel bytes")
-    _lib.call("voom_byteplane_merge", lo, hi, out, n, _stream(stream))
+    _lib.call("voom_byteplane_merge", _ptr(lo), _ptr(hi), _ptr(out), n, _stream(stream))
     return out
 
 
@@ -428,8 +440,8 @@ def byteplane_split_slots(pool: torch.Tensor, slots: torch.Tensor, lo: torch.Ten
     _require(lo.numel() >= n * slot_bytes // 2 and hi.numel() >= n * slot_bytes // 2,
              "plane buffers too small")
     _check_sums(sums, n)
-    _lib.call("voom_byteplane_split_slots", pool, slots, n, slot_bytes, num_slots,
-              lo, hi, sums, _stream(stream))
+    _lib.call("voom_byteplane_split_slots", _ptr(pool), _ptr(slots), n, slot_bytes, num_slots,
+              _ptr(lo), _ptr(hi), _ptr(sums), _stream(stream))
 
 
 def byteplane_merge_slots(lo: torch.Tensor, hi: torch.Tensor, pool: torch.Tensor,
@@ -446,8 +458,8 @@ def byteplane_merge_slots(lo: torch.Tensor, hi: torch.Tensor, pool: torch.Tensor
     _require(lo.numel() >= n * slot_bytes // 2 and hi.numel() >= n * slot_bytes // 2,
              "plane buffers too small")
     _check_sums(sums, n)
-    _lib.call("voom_byteplane_merge_slots", lo, hi, pool, slots, n,
-              slot_bytes, num_slots, sums, _stream(stream))
+    _lib.call("voom_byteplane_merge_slots", _ptr(lo), _ptr(hi), _ptr(pool), _ptr(slots), n,
+              slot_bytes, num_slots, _ptr(sums), _stream(stream))
 
 
 def _check_sums(sums: torch.Tensor | None, n: int) -> None:
@@ -465,8 +477,8 @@ def page_sums_verify(expected: torch.Tensor, got: torch.Tensor, tag: int,
              "checksums and status must be int32")
     _require(expected.numel() == got.numel() and status.numel() >= 2, "checksum sizes differ")
     _require(tag != 0, "tag must be non-zero")
-    _lib.call("voom_page_sums_verify", expected, got, expected.numel(), int(tag),
-              status, _stream(stream))
+    _lib.call("voom_page_sums_verify", _ptr(expected), _ptr(got), expected.numel(), int(tag),
+              _ptr(status), _stream(stream))
 
 
 def copy_rows(dst: int, dst_pitch: int, src: int, src_pitch: int, width: int, rows: int, *,
@@ -531,8 +543,8 @@ def spill_record(pools: list[torch.Tensor], slots: torch.Tensor, record: torch.T
     voom_spill_record documents."""
     rec_slots = slots.numel() if rec_slots is None else int(rec_slots)
     ptrs, sbytes, counts = _record_call_args(pools, slots, record, rec_slots, first, sums)
-    _lib.call("voom_spill_record", ctypes.addressof(ptrs), ctypes.addressof(sbytes),
-              ctypes.addressof(counts), len(pools), slots, slots.numel(), record,
+    _lib.call("voom_spill_record", ctypes.cast(ptrs, ctypes.c_void_p), ctypes.addressof(sbytes),
+              ctypes.addressof(counts), len(pools), _ptr(slots), slots.numel(), _ptr(record),
               rec_slots, int(first), int(bool(sums)), _stream(stream))
 
 
@@ -549,10 +561,10 @@ def reload_record(record: torch.Tensor, pools: list[torch.Tensor], slots: torch.
     if tag:
         _require(status is not None and status.is_cuda and status.dtype == torch.int32
                  and status.numel() >= 2, "a tag needs a device int32 status of 2 words")
-    _lib.call("voom_reload_record", record, rec_slots, int(first),
-              ctypes.addressof(ptrs), ctypes.addressof(sbytes),
-              ctypes.addressof(counts), len(pools), slots, slots.numel(), int(tag),
-              status if tag else None, _stream(stream))
+    _lib.call("voom_reload_record", _ptr(record), rec_slots, int(first),
+              ctypes.cast(ptrs, ctypes.c_void_p), ctypes.addressof(sbytes),
+              ctypes.addressof(counts), len(pools), _ptr(slots), slots.numel(), int(tag),
+              _ptr(status) if tag else None, _stream(stream))
 
 
 def slot_codec_supported(pool: torch.Tensor) -> bool:
@@ -564,7 +576,7 @@ def slot_codec_supported(pool: torch.Tensor) -> bool:
 
 
 def mla_workspace_bytes(batch: int, num_heads: int, num_ranges: int = 0) -> int:
-    return int(_lib.calls().voom_mla_workspace_bytes(batch, num_heads, num_ranges))
+    return int(_lib.lib().voom_mla_workspace_bytes(batch, num_heads, num_ranges))
 
 
 def mla_latent_decode(q_lat: torch.Tensor, lat_pool: torch.Tensor, block_table: torch.Tensor,
@@ -596,8 +608,8 @@ def mla_latent_decode(q_lat: torch.Tensor, lat_pool: torch.Tensor, block_table: 
     if out is None:
         out = torch.empty((B, H, 512), dtype=torch.bfloat16, device=dev)
     lse = torch.empty((B, H), dtype=torch.float32, device=dev) if return_lse else None
-    _lib.call("voom_mla_absorbed_decode", q_lat, lat_pool, block_table,
-              ctx_lens, out, lse, ws, need, B, H, LD, 512, PT,
+    _lib.call("voom_mla_absorbed_decode", _ptr(q_lat), _ptr(lat_pool), _ptr(block_table),
+              _ptr(ctx_lens), _ptr(out), _ptr(lse), _ptr(ws), need, B, H, LD, 512, PT,
               block_table.shape[1], slots, float(scale), int(num_ranges), _stream(stream))
     return (out, lse) if return_lse else out
 
@@ -627,15 +639,15 @@ def mla_sparse_decode(q_lat: torch.Tensor, lat_pool: torch.Tensor, block_table: 
              "block_table [B, max_pages], sel [B, k], sel_lens [B]")
     if _BOUNDS_CHECKS:
         check_selection(sel, sel_lens, block_table, slots, PT, stream=stream)
-    need = int(_lib.calls().voom_mla_sparse_workspace_bytes(B, H, sel.shape[1], int(num_ranges)))
+    need = int(_lib.lib().voom_mla_sparse_workspace_bytes(B, H, sel.shape[1], int(num_ranges)))
     if ws is None:
         ws = workspace(dev, need, tag=2)
     _require(ws.numel() * ws.element_size() >= need, "workspace too small")
     if out is None:
         out = torch.empty((B, H, 512), dtype=torch.bfloat16, device=dev)
     lse = torch.empty((B, H), dtype=torch.float32, device=dev) if return_lse else None
-    _lib.call("voom_mla_sparse_decode", q_lat, lat_pool, block_table,
-              sel, sel_lens, out, lse, ws, need, B, H, LD, 512, PT,
+    _lib.call("voom_mla_sparse_decode", _ptr(q_lat), _ptr(lat_pool), _ptr(block_table),
+              _ptr(sel), _ptr(sel_lens), _ptr(out), _ptr(lse), _ptr(ws), need, B, H, LD, 512, PT,
               block_table.shape[1], slots, sel.shape[1], float(scale), int(num_ranges),
               _stream(stream))
     return (out, lse) if return_lse else out
@@ -663,8 +675,8 @@ def dsa_index_scores(q_idx: torch.Tensor, w_head: torch.Tensor, k_idx: torch.Ten
     if out is None:
         out = torch.empty((B, cap), dtype=torch.float32, device=dev)
     _require(tuple(out.shape) == (B, cap) and out.dtype == torch.float32, "scores [B, cap] fp32")
-    _lib.call("voom_dsa_index_scores", q_idx, w_head, k_idx, lens,
-              out, B, NH, D, cap, float(scale), _stream(stream))
+    _lib.call("voom_dsa_index_scores", _ptr(q_idx), _ptr(w_head), _ptr(k_idx), _ptr(lens),
+              _ptr(out), B, NH, D, cap, float(scale), _stream(stream))
     return out
 
 
@@ -686,9 +698,9 @@ def dsa_topk(scores: torch.Tensor, lens: torch.Tensor, k: int, *,
         sel_lens = torch.empty((B,), dtype=torch.int32, device=dev)
     _require(sel.dtype == sel_lens.dtype == torch.int32 and tuple(sel.shape) == (B, int(k))
              and tuple(sel_lens.shape) == (B,), "sel [B, k] and sel_lens [B] int32")
-    need = int(_lib.calls().voom_dsa_topk_workspace_bytes(B, cap))
+    need = int(_lib.lib().voom_dsa_topk_workspace_bytes(B, cap))
     ws = workspace(dev, need, tag=4)
-    _lib.call("voom_dsa_topk", scores, lens, sel, sel_lens, ws,
+    _lib.call("voom_dsa_topk", _ptr(scores), _ptr(lens), _ptr(sel), _ptr(sel_lens), _ptr(ws),
               need, B, cap, int(k), _stream(stream))
     return sel, sel_lens
 
@@ -705,7 +717,7 @@ def add_rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float,
     _require(delta is None or (delta.shape == x.shape and delta.dtype == x.dtype), "delta like x")
     if out is None:
         out = torch.empty_like(x)
-    _lib.call("voom_add_rms_norm", x, delta, weight, out,
+    _lib.call("voom_add_rms_norm", _ptr(x), _ptr(delta), _ptr(weight), _ptr(out),
               x.numel() // H, H, float(eps), _stream(stream))
     return out
 
@@ -722,7 +734,7 @@ def rope_split(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, num_q_he
     q = torch.empty((B, num_q_heads, L, head_dim), dtype=qkv.dtype, device=dev)
     k = torch.empty((B, num_kv_heads, L, head_dim), dtype=qkv.dtype, device=dev)
     v = torch.empty_like(k)
-    _lib.call("voom_rope_split", qkv, cos, sin, q, k, v,
+    _lib.call("voom_rope_split", _ptr(qkv), _ptr(cos), _ptr(sin), _ptr(q), _ptr(k), _ptr(v),
               B, L, num_q_heads, num_kv_heads, head_dim, _stream(stream))
     return q, k, v
 
@@ -733,7 +745,7 @@ def silu_mul(gate_up: torch.Tensor, stream: torch.cuda.Stream | None = None) -> 
     _require(gate_up.dtype == torch.bfloat16 and gate_up.shape[-1] % 2 == 0, "bf16 [..., 2I]")
     inter = gate_up.shape[-1] // 2
     out = torch.empty((*gate_up.shape[:-1], inter), dtype=gate_up.dtype, device=dev)
-    _lib.call("voom_silu_mul", gate_up, out, gate_up.numel() // (2 * inter), inter,
+    _lib.call("voom_silu_mul", _ptr(gate_up), _ptr(out), gate_up.numel() // (2 * inter), inter,
               _stream(stream))
     return out
 
@@ -778,8 +790,8 @@ def gemv(x: torch.Tensor, weight: torch.Tensor, *, swiglu: bool = False,
     n = weight.shape[0] // 2 if swiglu else weight.shape[0]
     _require(not swiglu or weight.shape[0] % 2 == 0, "swiglu weight rows must be even")
     y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=dev)
-    _lib.call("voom_add_rms_norm_gemv", x, delta, ln_weight, float(eps),
-              x_out, weight, y, n, K, int(swiglu), _stream(stream))
+    _lib.call("voom_add_rms_norm_gemv", _ptr(x), _ptr(delta), _ptr(ln_weight), float(eps),
+              _ptr(x_out), _ptr(weight), _ptr(y), n, K, int(swiglu), _stream(stream))
     return y
 
 
@@ -803,8 +815,8 @@ def lm_head_argmax(x: torch.Tensor, weight: torch.Tensor, token: torch.Tensor, *
         _require(t is None or (t.dtype == torch.int64 and t.numel() >= 1), "int64 token outputs")
     need = 8 * ((N + 15) // 16)
     ws = workspace(dev, need, tag=5)
-    _lib.call("voom_lm_head_argmax", x, delta, ln_weight, float(eps),
-              weight, N, K, ws, ws.numel(), token, token_copy,
+    _lib.call("voom_lm_head_argmax", _ptr(x), _ptr(delta), _ptr(ln_weight), float(eps),
+              _ptr(weight), N, K, _ptr(ws), ws.numel(), _ptr(token), _ptr(token_copy),
               _stream(stream))
     return token
 
@@ -839,9 +851,9 @@ def qkv_rope_append(x: torch.Tensor, w_qkv: torch.Tensor, cos: torch.Tensor, sin
     _require(block_table.dtype == position.dtype == torch.int32 and block_table.dim() == 2,
              "int32 block_table [B, max_pages] and position")
     q = torch.empty((1, nq, 1, hd), dtype=x.dtype, device=dev)
-    _lib.call("voom_qkv_rope_append", w_qkv, x, delta, ln_weight,
-              float(eps), x_out, cos, sin, q,
-              k_pool, v_pool, block_table, position, nq, nkv, hd, K, PT,
+    _lib.call("voom_qkv_rope_append", _ptr(w_qkv), _ptr(x), _ptr(delta), _ptr(ln_weight),
+              float(eps), _ptr(x_out), _ptr(cos), _ptr(sin), _ptr(q),
+              _ptr(k_pool), _ptr(v_pool), _ptr(block_table), _ptr(position), nq, nkv, hd, K, PT,
               block_table.shape[1], slots, rope_rows, _stream(stream))
     return q
 
@@ -854,7 +866,7 @@ def linear_rows(x: torch.Tensor, weight: torch.Tensor, *,
     _require(weight.dim() == 2 and x.shape[-1] == weight.shape[1], "weight [N, K] with K = x's")
     n, K = weight.shape
     y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=dev)
-    _lib.call("voom_linear_rows", x, weight, y, x.numel() // max(K, 1), n, K,
+    _lib.call("voom_linear_rows", _ptr(x), _ptr(weight), _ptr(y), x.numel() // max(K, 1), n, K,
               _stream(stream))
     return y
 
@@ -871,8 +883,8 @@ def norm_swiglu_rows(x: torch.Tensor, weight: torch.Tensor, ln_weight: torch.Ten
              "weight [2I, K] with K = x's")
     n, K = weight.shape[0] // 2, weight.shape[1]
     y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=dev)
-    _lib.call("voom_norm_swiglu_rows", x, delta, ln_weight, float(eps),
-              x_out, weight, y, x.numel() // max(K, 1), n, K, _stream(stream))
+    _lib.call("voom_norm_swiglu_rows", _ptr(x), _ptr(delta), _ptr(ln_weight), float(eps),
+              _ptr(x_out), _ptr(weight), _ptr(y), x.numel() // max(K, 1), n, K, _stream(stream))
     return y
 
 
@@ -902,9 +914,9 @@ def qkv_rope_append_rows(x: torch.Tensor, w_qkv: torch.Tensor, cos: torch.Tensor
     _require(block_table.dtype == torch.int32 and block_table.dim() == 2
              and block_table.shape[0] == B, "block_table must be int32 [B, max_pages]")
     q = torch.empty((B, nq, L, hd), dtype=x.dtype, device=dev)
-    _lib.call("voom_qkv_rope_append_rows", w_qkv, x, delta, ln_weight,
-              float(eps), x_out, cos, sin, q, k_pool, v_pool,
-              block_table, B, L, int(start), nq, nkv, hd, K, PT, block_table.shape[1], slots,
+    _lib.call("voom_qkv_rope_append_rows", _ptr(w_qkv), _ptr(x), _ptr(delta), _ptr(ln_weight),
+              float(eps), _ptr(x_out), _ptr(cos), _ptr(sin), _ptr(q), _ptr(k_pool), _ptr(v_pool),
+              _ptr(block_table), B, L, int(start), nq, nkv, hd, K, PT, block_table.shape[1], slots,
               _stream(stream))
     return q
 
@@ -937,7 +949,7 @@ class HeadWeights:
         self.packed = torch.empty(nbytes // 2, dtype=torch.bfloat16, device=dev)
         if side is not None:
             side.wait_stream(torch.cuda.current_stream())  # w (and its copy) are ready
-        _lib.call("voom_mla_pack_head_weights", w, self.packed, self.heads, self.k,
+        _lib.call("voom_mla_pack_head_weights", _ptr(w), _ptr(self.packed), self.heads, self.k,
                   self.n, _stream(stream))
         _used_on(side, w, self.packed)
 
@@ -970,7 +982,7 @@ def mla_absorb_query(q_nope: torch.Tensor, q_rope: torch.Tensor, w_uk):
              "W_UK must be [H, dn, C] for q_nope [B, H, dn]")
     C, dr = w_uk.n, q_rope.shape[-1]
     q_lat = torch.empty((B, H, C + dr), dtype=q_nope.dtype, device=dev)
-    _lib.call("voom_mla_absorb_query", q_nope, q_rope, w_uk.packed, q_lat,
+    _lib.call("voom_mla_absorb_query", _ptr(q_nope), _ptr(q_rope), _ptr(w_uk.packed), _ptr(q_lat),
               B, H, dn, C, dr, _stream(None))
     return q_lat
 
@@ -1006,7 +1018,7 @@ def mla_absorb_query_tokens(q_nope: torch.Tensor, q_rope: torch.Tensor,
     q_nope, q_rope = _token_rows(q_nope), _token_rows(q_rope)
     q_lat = torch.empty((B * L, H, w_uk.n + dr), dtype=torch.bfloat16, device=q_nope.device)
     sx, st = q_nope.stride(), q_rope.stride()
-    _lib.call("voom_mla_head_rows", q_nope, q_rope, w_uk.packed, q_lat, B,
+    _lib.call("voom_mla_head_rows", _ptr(q_nope), _ptr(q_rope), _ptr(w_uk.packed), _ptr(q_lat), B,
               L, H, dn, w_uk.n, sx[0], sx[2], sx[1], dr, st[0], st[2], st[1], w_uk.n + dr,
               _stream(None))
     return q_lat
@@ -1020,7 +1032,7 @@ def mla_project_rows(wc: torch.Tensor, w_uv: HeadWeights) -> torch.Tensor:
     R, H, C = wc.shape
     _require(w_uv.heads == H and w_uv.k == C, "W_UV^T must be [H, C, dv] for weighted_c")
     out = torch.empty((R, H, w_uv.n), dtype=torch.bfloat16, device=wc.device)
-    _lib.call("voom_mla_head_rows", wc, None, w_uv.packed, out, 1, R, H, C,
+    _lib.call("voom_mla_head_rows", _ptr(wc), None, _ptr(w_uv.packed), _ptr(out), 1, R, H, C,
               w_uv.n, R * H * C, H * C, C, 0, 0, 0, 0, w_uv.n, _stream(None))
     return out
 
@@ -1059,7 +1071,7 @@ def head_gemv(x: torch.Tensor, w, *, out: torch.Tensor | None = None,
     side = _side_stream(stream)
     if side is not None:
         side.wait_stream(torch.cuda.current_stream())  # x's contiguous copy and out are ready
-    _lib.call("voom_mla_head_gemv", x, w.packed, out, B, H, K, N, K,
+    _lib.call("voom_mla_head_gemv", _ptr(x), _ptr(w.packed), _ptr(out), B, H, K, N, K,
               out.shape[2], _stream(stream))
     _used_on(side, x, out)
     return out
@@ -1098,8 +1110,8 @@ def mla_latent_decode_project(q_lat: torch.Tensor, lat_pool: torch.Tensor,
     y = torch.empty((B, H, w_uv.n), dtype=torch.bfloat16, device=dev)
     wc = torch.empty((B, H, 512), dtype=torch.bfloat16, device=dev) if return_weighted_c else None
     lse = torch.empty((B, H), dtype=torch.float32, device=dev) if return_lse else None
-    _lib.call("voom_mla_absorbed_decode_project", q_lat, lat_pool, block_table,
-              ctx_lens, w_uv.packed, w_uv.n, y, wc, lse, ws,
+    _lib.call("voom_mla_absorbed_decode_project", _ptr(q_lat), _ptr(lat_pool), _ptr(block_table),
+              _ptr(ctx_lens), _ptr(w_uv.packed), w_uv.n, _ptr(y), _ptr(wc), _ptr(lse), _ptr(ws),
               need, B, H, LD, 512, PT, block_table.shape[1], slots, float(scale), int(num_ranges),
               _stream(stream))
     _used_on(_side_stream(stream), y, wc, lse, ws)
@@ -1145,7 +1157,7 @@ def append_rows(src: torch.Tensor, pool: torch.Tensor, block_table: torch.Tensor
     _require(block_table.dtype == torch.int32 and positions.dtype == torch.int32
              and block_table.shape[0] == B and tuple(positions.shape) == (B,),
              "block_table [B, max_pages] and positions [B] must be int32")
-    _lib.call("voom_append_rows", src, pool, block_table, positions, B, L,
+    _lib.call("voom_append_rows", _ptr(src), _ptr(pool), _ptr(block_table), _ptr(positions), B, L,
               W, PT, block_table.shape[1], slots, _stream(stream))
 
 
@@ -1157,7 +1169,7 @@ def gather_rows(pool: torch.Tensor, block_table: torch.Tensor, seq_len: int, *,
     B = block_table.shape[0]
     _require(block_table.dtype == torch.int32, "block_table must be int32")
     out = torch.empty((B, seq_len, W), dtype=pool.dtype, device=dev)
-    _lib.call("voom_gather_rows", pool, block_table, out, B, seq_len, W, PT,
+    _lib.call("voom_gather_rows", _ptr(pool), _ptr(block_table), _ptr(out), B, seq_len, W, PT,
               block_table.shape[1], slots, _stream(stream))
     return out
 
@@ -1186,7 +1198,7 @@ def position_free_workspace_bytes(batch: int, num_q_heads: int, num_queries: int
                                   num_kv_heads: int, head_dim: int, num_keys: int,
                                   dtype: torch.dtype = torch.bfloat16,
                                   num_splits: int = 0) -> int:
-    return int(_lib.calls().voom_position_free_workspace_bytes(
+    return int(_lib.lib().voom_position_free_workspace_bytes(
         batch, num_q_heads, num_queries, num_kv_heads, head_dim, num_keys, DTYPE_CODES[dtype],
         num_splits))
 
@@ -1243,9 +1255,9 @@ def position_free_paged_attention(q: torch.Tensor, k_pages: torch.Tensor, v_page
     need = position_free_workspace_bytes(B, NQ, TQ, NKV, D, TK, q.dtype, num_splits)
     ws = workspace(q.device, need, tag=3)
     out = torch.empty_like(q)
-    _lib.call("voom_position_free_attention", q, k_pages, v_pages,
-              block_table, key_positions, query_positions, cos,
-              sin, out, ws, need, B, NQ, TQ, NKV, D, BLOCK, P, TK,
+    _lib.call("voom_position_free_attention", _ptr(q), _ptr(k_pages), _ptr(v_pages),
+              _ptr(block_table), _ptr(key_positions), _ptr(query_positions), _ptr(cos),
+              _ptr(sin), _ptr(out), _ptr(ws), need, B, NQ, TQ, NKV, D, BLOCK, P, TK,
               cos.shape[0], DTYPE_CODES[q.dtype], DTYPE_CODES[cos.dtype], float(scale),
               int(num_splits), _stream(stream))
     return out
