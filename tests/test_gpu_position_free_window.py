@@ -146,3 +146,36 @@ def test_weak_keys_keep_their_weight_in_fp16():
         args = (q, kp, vp, table, table, qpos, cos, sin)
         out = ops.position_free_paged_attention(*args, scale=1.0)
         check(out, reference(*args, 1.0), torch.float16)
+
+
+def slow_pair(dtype, TK, TQ, scores, values):
+    """One kv head of 128 dims with two query heads.  The queries hold 1 in the
+    slowest rotary pair, so that a key with s in its first dim scores s (its
+    rotation is small); ``scores`` and ``values`` [TK, 128] fill K and V."""
+    D = 128
+    q = torch.zeros((1, 2, TQ, D), dtype=dtype, device="cuda")
+    q[..., D // 2 - 1] = 1.0
+    q[..., D - 1] = 2.0 ** -14  # the partner dim, so that infinities there keep their sign
+    kp = torch.zeros((TK, 1, 1, D), dtype=dtype, device="cuda")
+    kp[:, 0, 0, D // 2 - 1] = torch.as_tensor(scores, device="cuda").to(dtype)
+    vp = values.to(dtype).reshape(TK, 1, 1, D)
+    table = torch.arange(TK, dtype=torch.int32, device="cuda")
+    qpos = torch.full((TQ,), TK + 1, dtype=torch.int32, device="cuda")
+    cos, sin = ops.rope_cache(TK + 2, D, 1e4, device="cuda")
+    return q, kp, vp, table, table + 1, qpos, cos, sin
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("first,count,splits", [(0, 200, 1), (0, 64, 0), (1000, 700, 3)])
+def test_keys_pushed_to_minus_infinity(dtype, first, count, splits):
+    """Whole tiles of visible keys that score -inf, at the start of a split too,
+    weigh nothing."""
+    print(f"[pf-window] -inf keys {dtype} {first} + {count}, splits={splits}", flush=True)
+    TK = 2000
+    g = torch.Generator(device="cuda").manual_seed(4)
+    scores = torch.randn(TK, generator=g, device="cuda")
+    scores[first:first + count] = -float("inf")
+    args = slow_pair(dtype, TK, staged_from(1, 2, 1, 128, TK), scores,
+                     torch.randn((TK, 128), generator=g, device="cuda"))
+    out = ops.position_free_paged_attention(*args, scale=1.0, num_splits=splits)
+    check(out, reference(*args, 1.0), dtype)

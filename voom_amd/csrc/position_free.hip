@@ -1265,7 +1265,7 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
   // Tile t where every row of the wavefront sees all of tiles t and t + 1.
   auto whole_tile = [&](int t, const uint16_t* tile, uint16_t* next, const Scores& sc,
                         Scores& nx) {
-    const float mref = m;
+    const float mref = m == -INFINITY ? 0.f : m;  // every key so far scored -inf: P = 0
     Weights pk;
     u32x4 ring[kA];
 #pragma unroll
