@@ -4,8 +4,8 @@ point rotates them, and against the same call made one query at a time.
 
 Bars, relative L2 over the output: fp16 8e-4 (its own rounding is at most 2^-12 /
 sqrt(3) = 1.4e-4 per value and the rotated keys carry one fp16 rounding that can
-fall the other way than fp64's, 2^-11 of a key now and then; P is kept to 22
-bits), bf16 4e-3 (output and softmax weights rounded to bf16, 1.1e-3 each).
+fall the other way than fp64's, 2^-11 of a key now and then; P is as good as in
+32 bits), bf16 4e-3 (output and softmax weights rounded to bf16, 1.1e-3 each).
 """
 import pytest
 import torch
@@ -179,3 +179,86 @@ def test_keys_pushed_to_minus_infinity(dtype, first, count, splits):
                      torch.randn((TK, 128), generator=g, device="cuda"))
     out = ops.position_free_paged_attention(*args, scale=1.0, num_splits=splits)
     check(out, reference(*args, 1.0), dtype)
+
+
+@pytest.mark.parametrize("wide", [False, True])
+def test_infinite_values_in_fp16(wide):
+    """An infinite V under a positive weight of any size gives that infinity
+    (weights with an exact fp16 value, and far below fp16's range, among them),
+    infinities of both signs and NaN give NaN, and the other dims keep their
+    values."""
+    TK, inf = 4000, float("inf")
+    TQ = staged_from(1, 2, 1, 128, TK) if wide else 1
+    print(f"[pf-window] infinite values, {TQ} queries", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(6)
+    scores = torch.zeros(TK)  # equal scores: every weight is exactly 1
+    scores[40] = -60.0        # e^-60
+    values = torch.randn((TK, 128), generator=g, device="cuda")
+    plain = values.clone()
+    for key, dim, v in ((7, 3, inf), (100, 4, -inf), (3999, 5, inf), (40, 6, inf), (900, 7, -inf),
+                        (901, 7, -inf), (5, 8, inf), (3000, 8, -inf), (64, 9, float("nan"))):
+        values[key, dim] = v
+    args = slow_pair(torch.float16, TK, TQ, scores, values)
+    out = ops.position_free_paged_attention(*args, scale=1.0)
+    ref = reference(*slow_pair(torch.float16, TK, TQ, scores, plain), 1.0)
+    torch.cuda.synchronize()
+    for dim, v in ((3, inf), (4, -inf), (5, inf), (6, inf), (7, -inf)):
+        assert torch.all(out[..., dim] == v), dim
+    assert torch.isnan(out[..., 8:10]).all()
+    rest = [d for d in range(128) if not 3 <= d <= 9]
+    check(out[..., rest], ref[..., rest], torch.float16)
+
+
+@pytest.mark.parametrize("NQ,NKV,D,TK", [(28, 4, 128, 700), (16, 8, 64, 1500), (6, 2, 128, 900),
+                                         (8, 8, 128, 333)])
+def test_infinite_values_of_one_head(NQ, NKV, D, TK):
+    """Infinities in single kv heads: every query that sees the key, nothing else;
+    in the staged route also not the queries before it, a tile away or less."""
+    G = NQ // NKV
+    most = staged_from(1, NQ, NKV, D, TK)
+    for TQ in (1, min(most, TK - 10)):
+        print(f"[pf-window] infinite values NQ={NQ} NKV={NKV} D={D} TQ={TQ}", flush=True)
+        args = list(inputs(1, NQ, NKV, TQ, D, 1, TK, torch.float16, seed=TK))
+        args[3] = torch.arange(TK, dtype=torch.int32, device="cuda")
+        want = reference(*args, D ** -0.5)
+        late = TK - 3  # seen by the last three queries
+        args[2][5, NKV - 1, 0, D - 1] = float("inf")
+        args[2][late, 0, 0, 17] = -float("inf")
+        out = ops.position_free_paged_attention(*args, scale=D ** -0.5)
+        torch.cuda.synchronize()
+        assert torch.all(out[:, -G:, :, D - 1] == float("inf"))
+        sees = args[5] >= late
+        assert torch.all(out[:, :G, sees, 17] == -float("inf"))
+        if TQ > 1 and TQ == most:
+            assert torch.isfinite(out[:, :G, ~sees, 17]).all()
+        hit = torch.zeros_like(out, dtype=torch.bool)
+        hit[:, -G:, :, D - 1] = True
+        hit[:, :G, :, 17] = True
+        check(out.masked_fill(hit, 0.0), want.masked_fill(hit, 0.0), torch.float16)
+
+
+@pytest.mark.parametrize("wide", [False, True])
+def test_weights_of_fp16_pages_to_32_bits(wide):
+    """Two keys of a block with values +-2^15 whose weights differ by d = 2^-15 .. 2^-13 (all
+    others weigh nothing) leave 2^15 tanh(d / 2): what the weights' own rounding adds is not hidden by the
+    output's.  Bound, for the weight just below 1: the exponential 2^-24 (an ulp),
+    hi and lo halves 2^-24, the sums behind them as much again, times 2^14; fp16
+    output 2^-12 of the value; scores of this size are exact to 2^-37."""
+    TK = 4000
+    TQ = staged_from(1, 2, 1, 128, TK) if wide else 40
+    print(f"[pf-window] 32-bit weights, {TQ} queries", flush=True)
+    scores = torch.full((TK,), -200.0)
+    values = torch.zeros((TK, 128), device="cuda")
+    values[10], values[12] = 2.0 ** 15, -2.0 ** 15
+    steps = torch.linspace(1.0, 2.0, TQ, device="cuda").to(torch.float16)
+    for e in (-15, -14):
+        scores[10], scores[12] = 2.0 ** e, 0.0
+        q, *args = slow_pair(torch.float16, TK, TQ, scores, values)
+        q[..., 63] = steps
+        q[..., 127] = 0.0
+        out = ops.position_free_paged_attention(q, *args, scale=1.0)
+        ref = reference(q, *args, 1.0)
+        torch.cuda.synchronize()
+        off = (out.double() - ref).abs()
+        bound = 2.0 ** 14 * 3 * 2.0 ** -24 + ref.abs() * 2.0 ** -12
+        assert bool((off <= bound).all()), (e, (off / bound).max().item())

@@ -88,10 +88,12 @@ struct EF32 {
 };
 
 // 16-bit element types on the matrix cores.  widen / narrow convert two packed
-// values; weights() packs four softmax weights for P . V in kParts operands and
-// returns their sum: bf16 weights are rounded to bf16 and summed as rounded, fp16
-// weights keep 21 bits in two fp16 halves (hi + lo) and are summed in fp32, so
-// that P stays as good as the fp32 weights of the generic kernel.
+// values; weights() packs two or four softmax weights for P . V in kParts operands
+// and returns their sum: bf16 weights are rounded to bf16 and summed as rounded.
+// fp16 weights are two fp16 halves, hi + lo, both rounded to nearest: within 2^-24
+// of a weight near 1 (an ulp of fp32), as good as the fp32 weights of the generic
+// kernel; they are summed in fp32.  An infinite or NaN V needs the weight in one
+// piece (0 times infinity is NaN), see odd_halves.
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -101,6 +103,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 template <typename E> struct Mma;
 template <> struct Mma<EBf16> {
   static constexpr int kParts = 1;
+  static constexpr float kPScale = 1.f;
   __device__ __forceinline__ static f32x16 mma32(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
@@ -127,15 +130,17 @@ template <> struct Mma<EBf16> {
 };
 template <> struct Mma<EF16> {
   static constexpr int kParts = 2;
-  // p0, p1 >= 0 as hi + lo: hi rounded toward zero, the exact rest rounded toward
-  // zero again (v_cvt_pkrtz, v_fma_mix: six operations), 2^-21 of p in all.
+  // Weights are scaled by kPScale, so that the halves of small ones do not fall
+  // into fp16's subnormals; l carries the same factor.  (Multiplied: added to the
+  // exponent instead, 12 would cost a weight near 1 three bits.)
+  static constexpr float kPScale = 4096.f;
+  // p0, p1 >= 0 as hi + lo: hi to nearest, the exact rest to nearest
+  // (v_cvt_pk_f16_f32, v_fma_mix: four operations).
   __device__ __forceinline__ static void split(float p0, float p1, uint32_t (&w)[kParts]) {
-    w[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(p0, p1));
+    w[0] = narrow(p0, p1);
     const f16x2 hi = __builtin_bit_cast(f16x2, w[0]);
-    w[1] = __builtin_bit_cast(
-        uint32_t,
-        __builtin_amdgcn_cvt_pkrtz(__builtin_fmaf(static_cast<float>(hi[0]), -1.f, p0),
-                                   __builtin_fmaf(static_cast<float>(hi[1]), -1.f, p1)));
+    w[1] = narrow(__builtin_fmaf(static_cast<float>(hi[0]), -1.f, p0),
+                  __builtin_fmaf(static_cast<float>(hi[1]), -1.f, p1));
   }
   __device__ __forceinline__ static f32x16 mma32(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
@@ -167,6 +172,29 @@ template <> struct Mma<EF16> {
     return p[0] + p[1] + p[2] + p[3];
   }
 };
+
+// fp16 V with infinities or NaN: hi * inf + lo * inf is NaN where lo is 0 or
+// negative.  Such values count apart from the others, under whole_weight: 1 for any
+// positive weight, else the weight (0 or NaN).
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t odd_halves(uint32_t x) {
+  return ((x & 0x7c00u) == 0x7c00u ? 0xffffu : 0u) |
+         ((x & 0x7c000000u) == 0x7c000000u ? 0xffff0000u : 0u);
+}
+__device__ __forceinline__ u32x4 finite_part(u32x4 v) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] &= ~odd_halves(v[e]);
+  return v;
+}
+__device__ __forceinline__ float whole_weight(float p) { return p > 0.f ? 1.f : p; }
+// A zero half once some value so far was infinite or NaN (two operations a pair).
+__device__ __forceinline__ u16x2 note_odd(u32x4 v, u16x2 seen) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    seen = __builtin_elementwise_min(seen, __builtin_bit_cast(u16x2, ~v[e] & 0x7c007c00u));
+  return seen;
+}
 
 // Four consecutive table entries as loaded (raw) and as fp32 (cvt): the MFMA
 // kernel keeps the raw chunk in registers while it is in flight and converts
@@ -289,10 +317,6 @@ template <int D, int HW, typename E, typename TT>
 __global__ __launch_bounds__(HW * kWave) __attribute__((amdgpu_waves_per_eu(HW >= 4 ? 2 : 1)))
 void pf_attention_kernel(PfArgs a) {
   typedef Mma<E> MM;
-  // P of fp16 pages is scaled by 2^kPBias, so that the hi and lo halves of
-  // small weights do not fall into fp16's subnormals (out and l carry the same
-  // factor)
-  constexpr float kPBias = MM::kParts == 2 ? 12.f : 0.f;
   constexpr int KS = D / 32;     // k-steps of the score MFMA
   constexpr int HS = D / 64;     // k-steps in one rotary half
   constexpr int DT = D / 16;     // dim tiles of out^T
@@ -528,7 +552,7 @@ void pf_attention_kernel(PfArgs a) {
       float p[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        p[r] = x[t][r] == -INFINITY ? 0.f : fast_exp2(x[t][r] - m_new + kPBias);
+        p[r] = x[t][r] == -INFINITY ? 0.f : fast_exp2(x[t][r] - m_new) * MM::kPScale;
       uint32_t pw[MM::kParts][2];
       ps += MM::weights(p, pw);
 #pragma unroll
@@ -574,6 +598,71 @@ void pf_attention_kernel(PfArgs a) {
     mA = mB;
     pgB = pgC;
     psB = psC;
+  }
+
+  if constexpr (MM::kParts == 2) {
+    // An infinite or NaN V leaves nothing finite in its dim whatever its weight, but
+    // possibly the wrong one of them: the keys' infinities once more, under whole
+    // weights and the scores as above.  Rare and key by key.
+    float any = 0.f;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) any = __builtin_fmaf(acc[d][r], 0.f, any);
+    }
+    if (__builtin_amdgcn_ballot_w64(any != 0.f) != 0) {
+      f32x4 odd[DT] = {};
+      for (int key = blo * kKeys; key < min(bhi * kKeys, a.TK); ++key) {
+        int pg, ps, rlo, rhi, kp;
+        pf_key_load(a, key, pg, ps);
+        pf_key_finish(a, kvh, key, pg, ps, rlo, rhi, kp);
+        const size_t at = static_cast<size_t>(pf_row_of(rlo, rhi, lane)) * D;
+        u32x2 vv[DT];
+        uint32_t here = 0;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) {
+          vv[d] = *reinterpret_cast<const u32x2*>(vpg + at + 16 * d + 4 * g);
+          here |= odd_halves(vv[d][0]) | odd_halves(vv[d][1]);
+        }
+        if (__builtin_amdgcn_ballot_w64(here != 0) == 0) continue;
+        float s = 0.f;
+#pragma unroll
+        for (int st = 0; st < HS; ++st) {
+          const int dim = 32 * st + 8 * g;
+          const u32x4 lo = *reinterpret_cast<const u32x4*>(kpg + at + dim);
+          const u32x4 hi = *reinterpret_cast<const u32x4*>(kpg + at + dim + D / 2);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const size_t to = static_cast<size_t>(kp) * (D / 2) + dim + 4 * (e >> 1);
+            const f32x4 c = TC::cvt(TC::load(a.cos_t, to)), sn = TC::cvt(TC::load(a.sin_t, to));
+            const f32x2 x = MM::widen(lo[e]), y = MM::widen(hi[e]);
+            const f32x2 qa = MM::widen(qop[st][e]), qb = MM::widen(qop[st + HS][e]);
+            const int n = 2 * (e & 1);
+            const f32x2 ra = MM::widen(MM::narrow(x[0] * c[n] - y[0] * sn[n],
+                                                  x[1] * c[n + 1] - y[1] * sn[n + 1]));
+            const f32x2 rb = MM::widen(MM::narrow(y[0] * c[n] + x[0] * sn[n],
+                                                  y[1] * c[n + 1] + x[1] * sn[n + 1]));
+            s += ra[0] * qa[0] + ra[1] * qa[1] + rb[0] * qb[0] + rb[1] * qb[1];
+          }
+        }
+        s = wave_sum_across_groups(s) * a.scale_log2e;
+        const bool sees = ps <= qpos;
+        const float wt = s == -INFINITY ? 0.f : whole_weight(fast_exp2(s - m_run));
+#pragma unroll
+        for (int d = 0; d < DT; ++d) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const f32x2 v = MM::widen(vv[d][r >> 1] & odd_halves(vv[d][r >> 1]));
+            odd[d][r] += sees && v[r & 1] != 0.f ? wt * v[r & 1] : 0.f;
+          }
+        }
+      }
+#pragma unroll
+      for (int d = 0; d < DT; ++d) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[d][r] = odd[d][r] != 0.f ? odd[d][r] : acc[d][r];
+      }
+    }
   }
 
   const float l_tot = wave_sum_across_groups(l_lane);
@@ -877,6 +966,19 @@ __global__ __launch_bounds__(kRedWaves * kWave) void pf_reduce_kernel(PfArgs a,
     L = L * rescale + Lc;
     M = Mn;
   }
+  // Past the last split a lane reads that split's row once more, with weight 0: an
+  // infinity there has become NaN, so once more without those rows (rare).
+  float any = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) any = __builtin_fmaf(acc[e], 0.f, any);
+  if (__builtin_amdgcn_ballot_w64(any != 0.f) != 0) {
+    acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = r; i < cnt; i += kRedRows) {
+      const size_t p = (first + i) * a.NCP + n;
+      if (ml2[p].x != -INFINITY)
+        acc += *reinterpret_cast<const f32x4*>(a.part_o + p * D + dim0) * fast_exp2(ml2[p].x - M);
+    }
+  }
   // rows of one wave share M: the lanes of a column sum their rows
 #pragma unroll
   for (int x = kRedCols; x < kWave; x <<= 1) {
@@ -939,6 +1041,7 @@ struct WinArgs {
   uint16_t* v_blk;      // [NKV, nblk, D, 32]
   int32_t* pos;         // [nblk * 32] positions for the mask (INT_MAX past the last key)
   int2* span;           // [nblk] smallest and largest of them
+  int32_t* odd;         // [NKV, nblk] fp16: whether V holds an infinity or a NaN
   int nblk;             // 32-key blocks, even
   int R;                // rows of a kv head: B * TQ * G, the head fastest
   int row_tiles, splits;
@@ -992,11 +1095,16 @@ __global__ __launch_bounds__(256) void pf_stage_kernel(WinArgs w) {
   const uint16_t* kp = static_cast<const uint16_t*>(a.k_pages);
   const uint16_t* vp = static_cast<const uint16_t*>(a.v_pages);
   const size_t out = (static_cast<size_t>(kvh) * w.nblk + blk) * (kKeys * D);
+  u16x2 seen = {0xffff, 0xffff};
   for (int i = t; i < kChunks; i += 256) {
     const int key = i / (D / 8), c = i % (D / 8);
     const u32x4 z = {0u, 0u, 0u, 0u};
-    const u32x4 v = row[key] < 0 ? z : __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
-                                           vp + row[key] * D + 8 * c));
+    u32x4 v = row[key] < 0 ? z : __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
+                                     vp + row[key] * D + 8 * c));
+    if constexpr (MM::kParts == 2) {
+      seen = note_odd(v, seen);
+      v = finite_part(v);  // pf_window_kernel's add_odd brings the others
+    }
     *reinterpret_cast<u32x4*>(vs + key * kVs + 8 * c) = v;
   }
   for (int i = t; i < kPairs; i += 256) {
@@ -1028,7 +1136,12 @@ __global__ __launch_bounds__(256) void pf_stage_kernel(WinArgs w) {
     *reinterpret_cast<u32x4*>(o) = lo;
     *reinterpret_cast<u32x4*>(o + D / 2) = hi;
   }
-  __syncthreads();
+  if constexpr (MM::kParts == 2) {
+    const int odd = __syncthreads_or(seen[0] == 0 || seen[1] == 0);
+    if (t == 0) w.odd[kvh * w.nblk + blk] = odd;
+  } else {
+    __syncthreads();
+  }
   for (int i = t; i < kChunks; i += 256) {
     const int d = i >> 2, c = i & 3;
     u32x4 v;
@@ -1065,8 +1178,6 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
   constexpr int KS = D / 16;
   constexpr int DT = D / 32;
   constexpr int kA = kWinAhead;
-  // P of fp16 pages is scaled by 2^kPBias (see pf_attention_kernel)
-  constexpr float kPBias = MM::kParts == 2 ? 12.f : 0.f;
   // masks of __builtin_amdgcn_sched_group_barrier
   constexpr int kValu = 0x002, kMfma = 0x008, kVmemRead = 0x020, kDsRead = 0x100, kTrans = 0x400;
   static_assert(kPieces >= NW && (kLoads == 8 || kLoads == 4), "loads of a stage");
@@ -1112,6 +1223,8 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
   }
   // keys end (for this workgroup) with the last block that one of its rows sees
   int n_tiles;
+  int odd_blocks = 0;  // != 0: some block's V had an infinity or a NaN
+  const int32_t* odd = wa.odd + static_cast<size_t>(kvh) * wa.nblk;
   {
     int top = INT_MIN;
 #pragma unroll
@@ -1124,10 +1237,12 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
     for (int o = 32; o > 0; o >>= 1) top = max(top, __shfl_xor(top, o));
     for (int i = lane; i < wa.nblk; i += kWave) {
       if (i * kKeys < a.TK && wa.span[i].x <= top) last = i;
+      if (MM::kParts == 2) odd_blocks |= odd[i];
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) last = max(last, __shfl_xor(last, o));
     n_tiles = uniform(last + 2) >> 1;
+    odd_blocks = __builtin_amdgcn_ballot_w64(odd_blocks != 0) != 0;
   }
   const int t_lo = static_cast<int>(static_cast<long long>(split) * n_tiles / wa.splits);
   const int t_hi = static_cast<int>(static_cast<long long>(split + 1) * n_tiles / wa.splits);
@@ -1255,8 +1370,8 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
   auto form_p = [&](int e, const Scores& sc, float mref, Weights& pk) {
     const int j = e >> 3, n = 2 * (e & 7);
     uint32_t pw[MM::kParts];
-    l = MM::weights(fast_exp2(__builtin_fmaf(sc[j][n], wa.scale, kPBias - mref)),
-                    fast_exp2(__builtin_fmaf(sc[j][n + 1], wa.scale, kPBias - mref)), pw, l);
+    l = MM::weights(fast_exp2(__builtin_fmaf(sc[j][n], wa.scale, -mref)) * MM::kPScale,
+                    fast_exp2(__builtin_fmaf(sc[j][n + 1], wa.scale, -mref)) * MM::kPScale, pw, l);
 #pragma unroll
     for (int part = 0; part < MM::kParts; ++part)
       pk[part][2 * j + (n >> 3)][(n & 7) >> 1] = pw[part];
@@ -1290,7 +1405,7 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
         form_p(e, sc, mref, pk);
         __builtin_amdgcn_sched_group_barrier(kValu, 2, 0);
         __builtin_amdgcn_sched_group_barrier(kTrans, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(kValu, MM::kParts == 2 ? 8 : 2, 0);
+        __builtin_amdgcn_sched_group_barrier(kValu, MM::kParts == 2 ? 10 : 2, 0);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -1341,6 +1456,50 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
     }
   };
 
+  // Infinities and NaN in V of key kt, under the whole weights of the rows that see
+  // it: V from the pages (the staged V holds the finite values), the key's score
+  // once more.  Rare; key by key, since two tiles' worth of operands would cost the
+  // loops above their registers.
+  auto add_odd = [&](int kt) {
+    const int tb = kt / a.BLOCK;
+    int page = a.table[tb];
+    page = static_cast<unsigned>(page) < static_cast<unsigned>(a.P) ? page : 0;
+    const uint16_t* vr = static_cast<const uint16_t*>(a.v_pages) +
+                         ((static_cast<size_t>(page) * a.NKV + kvh) * a.BLOCK + (kt - tb * a.BLOCK)) * D;
+    uint32_t any = 0;
+#pragma unroll
+    for (int i = 0; i < D / kWave; ++i) any |= odd_halves(vr[i * kWave + lane]);
+    if (__builtin_amdgcn_ballot_w64(any != 0) == 0) return;
+    const uint16_t* kr = kseg + static_cast<size_t>(kt) * D + 8 * lh;  // (blocks are contiguous)
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+      const u32x4 kk = *reinterpret_cast<const u32x4*>(kr + 16 * i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const f32x2 x = MM::widen(kk[e]), y = MM::widen(qop[i][e]);
+        s = __builtin_fmaf(x[1], y[1], __builtin_fmaf(x[0], y[0], s));
+      }
+    }
+    s += __shfl_xor(s, 32);
+    const float ref = m == -INFINITY ? 0.f : m;
+    const float wt = whole_weight(fast_exp2(__builtin_fmaf(s, wa.scale, -ref)));
+    const bool sees = wa.pos[kt] <= qpos;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const u32x2 x = *reinterpret_cast<const u32x2*>(vr + 32 * d + 8 * i + 4 * lh);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t pair = x[e >> 1];
+          const f32x2 v = MM::widen(pair & odd_halves(pair));
+          acc[d][4 * i + e] += sees && v[e & 1] != 0.f ? wt * v[e & 1] : 0.f;
+        }
+      }
+    }
+  };
+
   Scores sc_a, sc_b;
   auto landed = [&]() {
     wait_vmem_all();
@@ -1381,6 +1540,13 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
     if (t + 2 < t_hi) load_stage(t + 2, tile_a);
     edge_tile(t + 1, tile_b, sc_a);
     t += 2;
+  }
+
+  if (MM::kParts == 2 && odd_blocks) {
+    for (int blk = 2 * t_lo; blk < 2 * t_hi; ++blk) {
+      if (uniform(odd[blk]) == 0 || uniform(wa.span[blk].x) > q_hi) continue;
+      for (int kt = blk * kKeys; kt < min((blk + 1) * kKeys, a.TK); ++kt) add_odd(kt);
+    }
   }
 
   const float lt = l + __shfl_xor(l, 32);
@@ -1492,7 +1658,7 @@ struct PfPlan {
   bool window;            // the window kernels
   int row_tiles, nblk;
   size_t o_bytes;         // the partial outputs' bytes (the statistics follow)
-  size_t stage_at, pos_at, span_at;  // window: the staged blocks in the workspace
+  size_t stage_at, pos_at, span_at, odd_at;  // window: the staged blocks in the workspace
   size_t ws_bytes;
 };
 
@@ -1533,7 +1699,8 @@ PfPlan pf_plan(int B, int NQ, int TQ, int NKV, int D, int TK, int dtype, int num
     const size_t blocks = static_cast<size_t>(NKV) * p.nblk;
     p.pos_at = p.stage_at + blocks * 2 * kKeys * D * sizeof(uint16_t);
     p.span_at = p.pos_at + align256(static_cast<size_t>(p.nblk) * kKeys * sizeof(int32_t));
-    p.ws_bytes = p.span_at + align256(static_cast<size_t>(p.nblk) * sizeof(int2));
+    p.odd_at = p.span_at + align256(static_cast<size_t>(p.nblk) * sizeof(int2));
+    p.ws_bytes = p.odd_at + align256(blocks * sizeof(int32_t));
     return p;
   }
   p.hw = NKV % 8 == 0 ? 8 : NKV % 4 == 0 ? 4 : NKV % 2 == 0 ? 2 : 1;
@@ -1564,6 +1731,7 @@ int launch_pf_window(const PfPlan& p, const PfArgs& a, char* ws, bool f32_tab, v
   w.v_blk = w.k_blk + blocks * kKeys * D;
   w.pos = reinterpret_cast<int32_t*>(ws + p.pos_at);
   w.span = reinterpret_cast<int2*>(ws + p.span_at);
+  w.odd = reinterpret_cast<int32_t*>(ws + p.odd_at);
   w.nblk = p.nblk;
   w.R = a.B * a.NC;
   w.row_tiles = p.row_tiles;
