@@ -302,11 +302,12 @@ int voom_dsa_topk(const float* scores, const int32_t* lens, int32_t* sel, int32_
  * _F32; the reference's T).  table_dtype: VOOM_DTYPE_F32 or dtype (the
  * reference's "FP32 or match the Q/K/V dtype", :210-211).  head_dim a
  * multiple of 32 up to 256 (the reference: any multiple of 32); any query
- * count and any num_q_heads / num_kv_heads.  bf16 at head_dim 64 or 128 runs
- * on MFMA; other element types and head dims on an fp32 VALU kernel.
+ * count and any num_q_heads / num_kv_heads.  bf16 and fp16 at head_dim 64 or 128
+ * run on MFMA; fp32 and other head dims on an fp32 VALU kernel.
  * num_splits splits each (batch, kv head)'s keys over workgroups (0 = library
  * default); the workspace must hold voom_position_free_workspace_bytes(...)
- * for the same values.  Page ids outside [0, num_pages) read page 0 and
+ * for the same values (calls of many queries stage the pages in it, up to a
+ * gigabyte of them).  Page ids outside [0, num_pages) read page 0 and
  * table rows are read at positions clamped to [0, max_position); callers
  * validate them (voom_check_position_free_pages does, see below).
  * ------------------------------------------------------------------------- */

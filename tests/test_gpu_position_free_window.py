@@ -262,3 +262,34 @@ def test_weights_of_fp16_pages_to_32_bits(wide):
         off = (out.double() - ref).abs()
         bound = 2.0 ** 14 * 3 * 2.0 ** -24 + ref.abs() * 2.0 ** -12
         assert bool((off <= bound).all()), (e, (off / bound).max().item())
+
+
+def test_staged_pages_are_not_kept():
+    """The staged copy of the pages is this call's own: the shared scratch does not
+    grow, and past a gigabyte the pages are walked instead."""
+    print("[pf-window] scratch", flush=True)
+    for dtype in (torch.bfloat16, torch.float16):
+        args = inputs(1, 28, 4, 250, 128, 1, 8000, dtype, seed=1)
+        before = {k: t.numel() for k, t in ops._WORKSPACES.items()}
+        ops.position_free_paged_attention(*args, scale=0.1)
+        torch.cuda.synchronize()
+        assert {k: t.numel() for k, t in ops._WORKSPACES.items()} == before
+    need = [ops.position_free_workspace_bytes(1, 32, 250, 8, 128, n) for n in (200_000, 1_000_000)]
+    assert need[0] > 4 * 200_000 * 8 * 128  # staged
+    assert need[1] < 1 << 30, need
+
+
+def test_windows_on_a_side_stream():
+    """A window enqueued on another stream while the current one goes on allocating
+    and computing: workspace and output keep their memory until it has run."""
+    print("[pf-window] side stream", flush=True)
+    args = inputs(1, 28, 4, 250, 128, 1, 8000, torch.float16, seed=2)
+    want = ops.position_free_paged_attention(*args, scale=0.1)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(5):
+        got = ops.position_free_paged_attention(*args, scale=0.1, stream=side)
+        junk = [torch.full((1 << 22,), 7.0, device="cuda") for _ in range(8)]
+        del junk
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))

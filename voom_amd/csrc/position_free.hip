@@ -1670,9 +1670,13 @@ struct PfPlan {
 // 64 columns 89 / 100; 2,000 keys: 32 columns 22.5 / 22.4, 64 columns 28.8 / 23.9;
 // 9q/3kv, D = 64, 20,000 keys: 72 columns 34.4 / 34.1, 144 columns 49 / 40; 500
 // keys: 300 columns 16 / 20.
+//
+// The staged copy of K and V is scratch of the call, so it is bounded: past
+// kWinMaxStage (262,144 keys of 8 heads of 128) the pages are walked.
+constexpr long long kWinMaxStage = 1LL << 30;
 bool window_pays(long long cols, int TK, int NKV, int D) {
   const long long elems = static_cast<long long>(TK) * NKV * D;
-  return cols >= 56 + elems / (1 << 19) && cols * elems >= 1LL << 26;
+  return 4 * elems <= kWinMaxStage && cols >= 56 + elems / (1 << 19) && cols * elems >= 1LL << 26;
 }
 
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }

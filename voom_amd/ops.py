@@ -1191,6 +1191,10 @@ def rope_cache(max_position: int, head_dim: int, theta: float, *,
     return torch.cos(angles).contiguous(), torch.sin(angles).contiguous()
 
 
+# (query, head of a group) columns up to which position-free pages are never staged
+# (window_pays in position_free.hip)
+POSITION_FREE_WALKED = 55
+
 DTYPE_CODES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}  # VOOM_DTYPE_*
 
 
@@ -1253,8 +1257,17 @@ def position_free_paged_attention(q: torch.Tensor, k_pages: torch.Tensor, v_page
         check_position_free_pages(block_table, key_positions, BLOCK, P, cos.shape[0],
                                   stream=stream)
     need = position_free_workspace_bytes(B, NQ, TQ, NKV, D, TK, q.dtype, num_splits)
-    ws = workspace(q.device, need, tag=3)
+    side = _side_stream(stream)
+    if side is not None or B * (NQ // NKV) * TQ > POSITION_FREE_WALKED:
+        # calls of many columns may keep a copy of the pages in their workspace
+        # (megabytes to a gigabyte): their own, given back when they have run, on
+        # the stream that uses it
+        with torch.cuda.stream(stream):
+            ws = torch.empty(max(need, 256), dtype=torch.uint8, device=q.device)
+    else:
+        ws = workspace(q.device, need, tag=3)
     out = torch.empty_like(q)
+    _used_on(side, out)
     _lib.call("voom_position_free_attention", _ptr(q), _ptr(k_pages), _ptr(v_pages),
               _ptr(block_table), _ptr(key_positions), _ptr(query_positions), _ptr(cos),
               _ptr(sin), _ptr(out), _ptr(ws), need, B, NQ, TQ, NKV, D, BLOCK, P, TK,
