@@ -1206,10 +1206,11 @@ __host__ __device__ __forceinline__ int range_groups(int NR) {
 __host__ __device__ __forceinline__ bool merges_in_groups(int B, int NR) {
   return NR > kSmallRanges && static_cast<long long>(B) * range_groups(NR) <= kMaxStates;
 }
-struct GroupState {
+struct alignas(16) GroupState {
   float o[kC];  // sum of the group's weighted rows, relative to M
   float M, L;
 };
+static_assert(sizeof(GroupState) % 16 == 0, "states are read and written as f32x4");
 __device__ __forceinline__ int group_count(int NR, int group) {
   const int left = NR - group * kSmallRanges;
   return left < kSmallRanges ? left : kSmallRanges;
@@ -1294,7 +1295,7 @@ constexpr int kRgThreads = 512;
 __global__ __launch_bounds__(kRgThreads) void mla_reduce_groups_kernel(
     const void* __restrict__ part_o, const float* __restrict__ part_ml,
     uint16_t* __restrict__ out, float* __restrict__ lse_out, int B, int H, int NR) {
-  __shared__ __attribute__((aligned(16))) GroupState st[kMaxStates];
+  __shared__ GroupState st[kMaxStates];
   const int lane = threadIdx.x & 63;
   const int w = uniform(threadIdx.x >> 6);
   const int task = blockIdx.x;
@@ -1337,7 +1338,7 @@ __global__ __launch_bounds__(kRpThreads) void mla_reduce_project_kernel(
     float* __restrict__ lse_out, int B, int H, int NR, int DV, int NT, int splits) {
   __shared__ __attribute__((aligned(16))) uint16_t wl[kRpPartTiles * kRpSteps * 512];
   __shared__ __attribute__((aligned(16))) uint16_t wcs[16][kC + 8];
-  __shared__ __attribute__((aligned(16))) GroupState states[GROUPED ? kMaxStates : 1];
+  __shared__ GroupState states[GROUPED ? kMaxStates : 1];
   // workgroups h + H part (same XCD for every part of a head when H % 8 == 0,
   // so the parts' reads of the head's partial rows meet in one L2) split the
   // head's column tiles; each merges all rows, part 0 writes weighted_c / lse
