@@ -406,3 +406,17 @@ def test_products_of_many_rows_have_the_decode_bits(B, L, H, K, N, dr):
     torch.cuda.synchronize()
     for y in got:
         assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
+
+
+def test_products_of_many_rows_refuse_queries_of_other_shapes():
+    """q_rope of fewer entries, heads or tokens than q_nope, and flat queries."""
+    print("[mla] head rows, refused shapes", flush=True)
+    w = ops.pack_head_weights(torch.zeros((4, 128, 512), dtype=torch.bfloat16, device="cuda"))
+    q = torch.zeros((2, 4, 20, 128), dtype=torch.bfloat16, device="cuda")
+    r = torch.zeros((2, 4, 20, 64), dtype=torch.bfloat16, device="cuda")
+    for bad in (r[:1], r[:, :3], r[:, :, :19], r[0], r[None]):
+        with pytest.raises(ValueError):
+            ops.mla_absorb_query_tokens(q, bad, w)
+    with pytest.raises(ValueError):
+        ops.mla_absorb_query_tokens(q[0], r[0], w)
+    assert ops.mla_absorb_query_tokens(q, r, w).shape == (40, 4, 576)

@@ -1012,6 +1012,8 @@ def mla_absorb_query_tokens(q_nope: torch.Tensor, q_rope: torch.Tensor,
     _require(q_nope.is_cuda and q_rope.device == q_nope.device == w_uk.packed.device,
              "q and W_UK must be on one ROCm device")
     _require(q_nope.dtype == q_rope.dtype == torch.bfloat16, "bf16 q_nope and q_rope")
+    _require(q_nope.dim() == q_rope.dim() == 4 and q_rope.shape[:3] == q_nope.shape[:3],
+             "q_nope [B, H, L, dn], q_rope [B, H, L, dr]")
     B, H, L, dn = q_nope.shape
     dr = q_rope.shape[-1]
     _require(w_uk.heads == H and w_uk.k == dn, "W_UK must be [H, dn, C] for q_nope")
