@@ -420,3 +420,21 @@ def test_products_of_many_rows_refuse_queries_of_other_shapes():
     with pytest.raises(ValueError):
         ops.mla_absorb_query_tokens(q[0], r[0], w)
     assert ops.mla_absorb_query_tokens(q, r, w).shape == (40, 4, 576)
+
+
+def test_one_sequence_with_any_batch_stride():
+    """A dimension of size 1 may carry any stride: a single sequence cut out of a
+    buffer whose rows are not a multiple of eight elements."""
+    print("[mla] head rows, odd strides of single entries", flush=True)
+    B, H, L, K, dr = 1, 4, 33, 128, 64
+    g = torch.Generator(device="cuda").manual_seed(9)
+    w = ops.pack_head_weights((torch.randn((H, K, 512), generator=g, device="cuda") * 0.05).to(
+        torch.bfloat16))
+    x = torch.randn((B, H, L, K), generator=g, device="cuda").to(torch.bfloat16)
+    t = torch.randn((B, H, L, dr), generator=g, device="cuda").to(torch.bfloat16)
+    want = ops.mla_absorb_query_tokens(x, t, w)
+    odd = [a.as_strided(a.shape, (a.numel() + 3, *a.stride()[1:])) for a in (x, t)]
+    assert odd[0].is_contiguous() and odd[0].stride(0) % 8
+    got = ops.mla_absorb_query_tokens(*odd, w)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))

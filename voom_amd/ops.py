@@ -994,14 +994,15 @@ def head_rows_supported(w: HeadWeights, tail: int = 0) -> bool:
             and (tail == 0 or tail % 8 == 0))
 
 
-def _token_rows(t: torch.Tensor) -> torch.Tensor:
-    """[B, H, L, D] as voom_mla_head_rows reads it: unit stride in D, the others
-    and the start 16-byte aligned (a copy where they are not)."""
-    if t.stride(3) != 1 or any(t.stride(i) % 8 for i in range(3)) or t.data_ptr() % 16:
-        t = t.contiguous()
-        if t.data_ptr() % 16:
-            t = t.clone()
-    return t
+def _token_rows(t: torch.Tensor) -> tuple[torch.Tensor, list[int]]:
+    """[B, H, L, D] as voom_mla_head_rows reads it, with the strides of B, H and L:
+    unit stride in D, the others and the start 16-byte aligned (a copy where they
+    are not; dimensions of size 1 have no stride to speak of)."""
+    strides = [0 if t.shape[i] == 1 else t.stride(i) for i in range(3)]
+    if t.stride(3) != 1 or any(s % 8 for s in strides) or t.data_ptr() % 16:
+        t = t.clone(memory_format=torch.contiguous_format)
+        strides = [t.stride(i) for i in range(3)]
+    return t, strides
 
 
 def mla_absorb_query_tokens(q_nope: torch.Tensor, q_rope: torch.Tensor,
@@ -1017,9 +1018,8 @@ def mla_absorb_query_tokens(q_nope: torch.Tensor, q_rope: torch.Tensor,
     B, H, L, dn = q_nope.shape
     dr = q_rope.shape[-1]
     _require(w_uk.heads == H and w_uk.k == dn, "W_UK must be [H, dn, C] for q_nope")
-    q_nope, q_rope = _token_rows(q_nope), _token_rows(q_rope)
+    (q_nope, sx), (q_rope, st) = _token_rows(q_nope), _token_rows(q_rope)
     q_lat = torch.empty((B * L, H, w_uk.n + dr), dtype=torch.bfloat16, device=q_nope.device)
-    sx, st = q_nope.stride(), q_rope.stride()
     _lib.call("voom_mla_head_rows", _ptr(q_nope), _ptr(q_rope), _ptr(w_uk.packed), _ptr(q_lat), B,
               L, H, dn, w_uk.n, sx[0], sx[2], sx[1], dr, st[0], st[2], st[1], w_uk.n + dr,
               _stream(None))
