@@ -347,12 +347,15 @@ def test_head_gemv_writes_into_a_wider_row_and_rejects_bad_shapes():
 
 
 @pytest.mark.parametrize("batch,nr", [(1, 17), (1, 40), (1, 128), (1, 384), (1, 400), (3, 128),
-                                      (2, 193), (7, 33), (16, 17)])
+                                      (2, 193), (7, 33), (16, 17), (4, 20), (5, 24), (6, 32),
+                                      (6, 33)])
 def test_merges_of_many_ranges(batch, nr):
-    """More than 16 ranges: merged in groups by several wavefronts while a
-    workgroup holds the groups' states (24: 1 x 384, 3 x 128, 7 x 33 and
-    16 x 17 lie on either side), else by one.  Both merging kernels give the
-    same bits, and the oracle's values (empty ranges among them)."""
+    """More than 16 ranges: merged in groups by several wavefronts, up to 24
+    groups in all (1 x 384 and 3 x 128, not 1 x 400 and 2 x 193) and 12 from five
+    sequences on (6 x 32, not 6 x 33, 7 x 33 and 16 x 17), else by one; two groups
+    with one, two and three rows to a workgroup (1 x 17, 4 x 20, 6 x 32).  Both
+    merging kernels give the same bits, and the oracle's values (empty ranges
+    among them)."""
     print(f"[mla] merge of {nr} ranges, batch {batch}", flush=True)
     ctx = [1500, 0, 700, 64, 65, 3, 900] + [130] * 9  # one of them empty
     inp = synthetic.mla_decode_inputs(batch=batch, heads=64, ctx_lens=ctx[:batch])

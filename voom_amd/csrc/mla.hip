@@ -1197,14 +1197,18 @@ __device__ __forceinline__ void combine_small_ranges(const SmallRanges& sr, int 
 // groups of kSmallRanges are merged by as many wavefronts, each in its one
 // memory round trip, and the groups' states meet in LDS in group order.  One
 // wavefront per sequence took a round trip per eight ranges (1 sequence, 128
-// ranges: 18 of 38 us).  The rule depends on (B, NR) only and both merging
-// kernels use it, so they give the same bits.
+// ranges: 18 of 38 us).  The eight wavefronts of the fused merge take a sequence each
+// anyway, so it gains less the more there are: 128 heads, 4 in 32 ranges 25.0 us one
+// wavefront each, 22.5 in groups; 64 heads, 6 in 32 21.6 and 21.0, but 8 in 24 20.6
+// and 21.8, 12 in 20 23.9 and 25.6.  The rule depends on (B, NR) only and both
+// merging kernels use it, so they give the same bits.
 constexpr int kMaxStates = 24;  // group states a workgroup of the fused merge can hold
 __host__ __device__ __forceinline__ int range_groups(int NR) {
   return (NR + kSmallRanges - 1) / kSmallRanges;
 }
 __host__ __device__ __forceinline__ bool merges_in_groups(int B, int NR) {
-  return NR > kSmallRanges && static_cast<long long>(B) * range_groups(NR) <= kMaxStates;
+  return NR > kSmallRanges &&
+         static_cast<long long>(B) * range_groups(NR) <= (B <= 4 ? kMaxStates : kMaxStates / 2);
 }
 struct alignas(16) GroupState {
   float o[kC];  // sum of the group's weighted rows, relative to M
@@ -1289,26 +1293,41 @@ __global__ __launch_bounds__(kThreads) void mla_reduce_kernel(
   if (lse_out != nullptr && lane == 0) lse_out[task] = merged_lse(M, L);
 }
 
-// mla_reduce_kernel<true> where merges_in_groups: one workgroup of eight
-// wavefronts per (sequence, head).
-constexpr int kRgThreads = 512;
-__global__ __launch_bounds__(kRgThreads) void mla_reduce_groups_kernel(
+// mla_reduce_kernel<true> where merges_in_groups: workgroups of eight wavefronts, one
+// per group of `rows` (sequence, head) rows, with the LDS of their states.  Two groups
+// leave six wavefronts over, so up to four rows share a workgroup, down to one
+// workgroup per two CUs.  Merge and latent kernel (which is slower behind many
+// workgroups) together, 128 heads, one wavefront per row / a workgroup per row / now:
+// 4 sequences in 24 ranges 19.2 / 20.3 / 19.3 us, 5 in 24 19.0 / 21.9 / 19.6, 6 in 20
+// 18.7 / 21.5 / 19.1; 1 in 32 15.7 / 15.3 / 15.3.  Three groups and more are faster a
+// workgroup per row: 2 in 48 20.9 / 20.9, shared 22.0; 1 in 128 29.0 / 22.9.
+constexpr int kRgWaves = 8;
+int rows_per_workgroup(int tasks, int groups) {
+  if (groups > 2) return 1;
+  const int rows = 2 * tasks / device_cu_count();
+  return rows < 1 ? 1 : rows > kRgWaves / groups ? kRgWaves / groups : rows;
+}
+__global__ __launch_bounds__(kRgWaves* kWave) void mla_reduce_groups_kernel(
     const void* __restrict__ part_o, const float* __restrict__ part_ml,
-    uint16_t* __restrict__ out, float* __restrict__ lse_out, int B, int H, int NR) {
-  __shared__ GroupState st[kMaxStates];
+    uint16_t* __restrict__ out, float* __restrict__ lse_out, int B, int H, int NR, int rows) {
+  extern __shared__ GroupState states[];  // [rows, groups]
   const int lane = threadIdx.x & 63;
   const int w = uniform(threadIdx.x >> 6);
-  const int task = blockIdx.x;
+  const int groups = range_groups(NR);
+  const int mine = rows == 1 ? 0 : w >> 1;  // this wavefront's row (two groups each)
+  const int task = blockIdx.x * rows + mine;
   const int b = task / H;
   const int h = task - b * H;
-  const int groups = range_groups(NR);
-  for (int g = w; g < groups; g += kRgThreads / kWave) {
-    SmallRanges sr;
-    load_group(part_o, part_ml, b, h, H, NR, g, lane, sr);
-    store_group(sr, NR, g, lane, &st[g]);
+  GroupState* st = states + mine * groups;
+  if (task < B * H) {
+    for (int g = w - mine * groups; g < groups; g += kRgWaves) {
+      SmallRanges sr;
+      load_group(part_o, part_ml, b, h, H, NR, g, lane, sr);
+      store_group(sr, NR, g, lane, &st[g]);
+    }
   }
   lds_barrier();
-  if (w != 0) return;
+  if (w != mine * groups || task >= B * H) return;
   f32x4 acc[kDPL / 4];
   float M, L;
   combine_groups(st, groups, lane, acc, M, L);
@@ -1485,9 +1504,14 @@ int launch_mla(const MlaArgs& a, int hg, bool sparse, long long grid, uint16_t* 
   if (rc) return rc;
   const unsigned red_grid = static_cast<unsigned>((a.B * a.H + 3) / 4);
   if (hg == 64 && merges_in_groups(a.B, a.NR)) {
-    hipLaunchKernelGGL(mla_reduce_groups_kernel, dim3(static_cast<unsigned>(a.B * a.H)),
-                       dim3(kRgThreads), 0, stream, static_cast<const void*>(a.part_o16), a.part_ml,
-                       out, lse_out, a.B, a.H, a.NR);
+    const int groups = range_groups(a.NR);
+    const int rows = rows_per_workgroup(a.B * a.H, groups);
+    const int waves = groups == 2 ? 2 * rows : kRgWaves;
+    hipLaunchKernelGGL(mla_reduce_groups_kernel,
+                       dim3(static_cast<unsigned>((a.B * a.H + rows - 1) / rows)),
+                       dim3(waves * kWave), groups * rows * sizeof(GroupState), stream,
+                       static_cast<const void*>(a.part_o16), a.part_ml, out, lse_out, a.B, a.H,
+                       a.NR, rows);
   } else if (hg == 64) {
     hipLaunchKernelGGL(mla_reduce_kernel<true>, dim3(red_grid), dim3(kThreads), 0, stream,
                        static_cast<const void*>(a.part_o16), a.part_ml, out, lse_out, a.B, a.H, a.NR);
