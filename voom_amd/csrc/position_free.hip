@@ -1223,8 +1223,6 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
   }
   // keys end (for this workgroup) with the last block that one of its rows sees
   int n_tiles;
-  int odd_blocks = 0;  // != 0: some block's V had an infinity or a NaN
-  const int32_t* odd = wa.odd + static_cast<size_t>(kvh) * wa.nblk;
   {
     int top = INT_MIN;
 #pragma unroll
@@ -1237,15 +1235,17 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
     for (int o = 32; o > 0; o >>= 1) top = max(top, __shfl_xor(top, o));
     for (int i = lane; i < wa.nblk; i += kWave) {
       if (i * kKeys < a.TK && wa.span[i].x <= top) last = i;
-      if (MM::kParts == 2) odd_blocks |= odd[i];
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) last = max(last, __shfl_xor(last, o));
     n_tiles = uniform(last + 2) >> 1;
-    odd_blocks = __builtin_amdgcn_ballot_w64(odd_blocks != 0) != 0;
   }
   const int t_lo = static_cast<int>(static_cast<long long>(split) * n_tiles / wa.splits);
   const int t_hi = static_cast<int>(static_cast<long long>(split + 1) * n_tiles / wa.splits);
+  // whether V of this workgroup's blocks 2 t_lo + lane, + 64 .. had infinities or NaN
+  const int32_t* odd = wa.odd + static_cast<size_t>(kvh) * wa.nblk;
+  int odd_blocks = 0;
+  if (MM::kParts == 2 && 2 * t_lo + lane < 2 * t_hi) odd_blocks = odd[2 * t_lo + lane];
 
   u32x4 qop[KS];
   auto load_q = [&]() {
@@ -1542,7 +1542,10 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
     t += 2;
   }
 
-  if (MM::kParts == 2 && odd_blocks) {
+  if constexpr (MM::kParts == 2) {
+    for (int i = 2 * t_lo + kWave + lane; i < 2 * t_hi; i += kWave) odd_blocks |= odd[i];
+  }
+  if (MM::kParts == 2 && __builtin_amdgcn_ballot_w64(odd_blocks != 0) != 0) {
     for (int blk = 2 * t_lo; blk < 2 * t_hi; ++blk) {
       if (uniform(odd[blk]) == 0 || uniform(wa.span[blk].x) > q_hi) continue;
       for (int kt = blk * kKeys; kt < min((blk + 1) * kKeys, a.TK); ++kt) add_odd(kt);
