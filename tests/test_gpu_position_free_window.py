@@ -70,12 +70,30 @@ def check(got, ref, dtype):
 
 
 def staged_from(B, NQ, NKV, D, TK):
-    """The fewest queries that take the staged route (window_pays in
-    position_free.hip): 56 columns plus one per 2^19 elements of K, and 2^26
-    columns times elements."""
+    """The fewest queries that take the staged route (kStageRules in
+    position_free.hip)."""
+    hw = next(h for h in (8, 4, 2, 1) if NKV % h == 0)
+    least, extra = {(64, 1): (48, 140), (64, 2): (110, 300), (64, 4): (72, 70), (64, 8): (65, 60),
+                    (128, 1): (48, 110), (128, 2): (65, 110), (128, 4): (56, 110),
+                    (128, 8): (56, 17)}[D, hw]
     elems = TK * NKV * D
-    cols = max(56 + elems // (1 << 19), -(-(1 << 26) // elems))
+    least += min(elems >> 19, 16) if (D, hw) == (128, 8) else 0
+    cols = least + -(-(extra << 19) // elems)
     return -(-cols // (B * (NQ // NKV)))
+
+
+def test_staged_from_is_the_rule():
+    """The workspace tells the routes apart: partials of many splits against the
+    staged pages."""
+    for B, NQ, NKV, D, TK in ((1, 28, 4, 128, 3000), (1, 32, 8, 128, 700), (1, 8, 8, 128, 9000), (2, 9, 3, 64, 5000),
+                              (1, 4, 2, 64, 8000), (1, 16, 2, 128, 900), (1, 8, 8, 64, 2000),
+                              (1, 12, 12, 64, 1500), (1, 7, 1, 128, 20000)):
+        TQ = staged_from(B, NQ, NKV, D, TK)
+        need = [ops.position_free_workspace_bytes(B, NQ, n, NKV, D, TK, num_splits=1)
+                for n in (TQ - 1, TQ)]
+        staged = 4 * -(-TK // 64) * 64 * NKV * D
+        assert need[0] < staged <= need[1], (need, staged)
+        assert ops._may_stage_pages(B * (NQ // NKV) * TQ, TK * NKV * D)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

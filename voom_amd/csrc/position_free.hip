@@ -1665,21 +1665,43 @@ struct PfPlan {
   size_t ws_bytes;
 };
 
-// Columns times keys from which staging the pages pays: the staged route costs a
-// pass over the pages (10 us at 4 MiB of K, 80 us at 64 MiB) and about 19 us of
-// launches and fill, the page-walking one a rotation of every key per 16 columns.
-// Measured (bf16, walking / staged, us): 28q/4kv, D = 128, 8,003 keys: 56 columns
-// 29.5 / 34.4, 112 columns 45 / 35, 1,750 columns 449 / 76; 32q/8kv, 32,768 keys:
-// 64 columns 89 / 100; 2,000 keys: 32 columns 22.5 / 22.4, 64 columns 28.8 / 23.9;
-// 9q/3kv, D = 64, 20,000 keys: 72 columns 34.4 / 34.1, 144 columns 49 / 40; 500
-// keys: 300 columns 16 / 20.
-//
+// kv heads of one workgroup of pf_attention_kernel.
+int heads_per_workgroup(int NKV) {
+  return NKV % 8 == 0 ? 8 : NKV % 4 == 0 ? 4 : NKV % 2 == 0 ? 2 : 1;
+}
+
+// Columns from which staging the pages pays.  The staged route takes about 21 us and
+// 1.2 us per 2^19 elements of K (a pass over the pages, launches and fill), hardly
+// growing with the columns; the page-walking one is short for few columns and grows
+// by a rotation of every key per 16 of them, at a rate of its own in each variant
+// (head dim, kv heads per workgroup).  So per variant: `least` columns however many
+// keys, and `extra` / e more with e = elements / 2^19, without which the walk is over
+// before the staged route's fixed part; eight heads of 128, whose workgroups just
+// fill the CUs at 64 columns, stay with the walk there from e = 8 on (`slope` 1: one
+// column more per e up to 16).  Measured with either route at 1,128 points of 10 head
+// geometries, 300 to 40,000 keys and 40 to 1,000 columns, bf16, walking / staged, us:
+// 9q/3kv, D = 64, 5,000 keys: 99 columns 20.1 / 23.1, 177 columns 24.4 / 24.8; 28q/4kv,
+// D = 128, 3,000 keys: 63 columns 21.9 / 26.2, 98 columns 28.7 / 27.4; 32q/8kv, 1,500
+// keys: 56 columns 20.7 / 21, 64 columns 24.5 / 21.9; 4q/2kv, D = 64, 12,000 keys: 120
+// columns 19.8 / 26.8, 200 columns 28 / 26.
+struct StageRule {
+  int least, extra, slope;
+};
+constexpr StageRule kStageRules[2][4] = {
+    // kv heads per workgroup: 1, 2, 4, 8
+    {{48, 140, 0}, {110, 300, 0}, {72, 70, 0}, {65, 60, 0}},  // D = 64
+    {{48, 110, 0}, {65, 110, 0}, {56, 110, 0}, {56, 17, 1}},  // D = 128
+};
 // The staged copy of K and V is scratch of the call, so it is bounded: past
 // kWinMaxStage (262,144 keys of 8 heads of 128) the pages are walked.
 constexpr long long kWinMaxStage = 1LL << 30;
 bool window_pays(long long cols, int TK, int NKV, int D) {
   const long long elems = static_cast<long long>(TK) * NKV * D;
-  return 4 * elems <= kWinMaxStage && cols >= 56 + elems / (1 << 19) && cols * elems >= 1LL << 26;
+  const StageRule r = kStageRules[D == 128][ilog2(heads_per_workgroup(NKV))];
+  const long long e = elems >> 19;
+  const long long least = r.least + r.slope * (e < 16 ? e : 16);
+  return 4 * elems <= kWinMaxStage && cols >= least &&
+         (cols - least) * elems >= static_cast<long long>(r.extra) << 19;
 }
 
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
@@ -1710,7 +1732,7 @@ PfPlan pf_plan(int B, int NQ, int TQ, int NKV, int D, int TK, int dtype, int num
     p.ws_bytes = p.odd_at + align256(blocks * sizeof(int32_t));
     return p;
   }
-  p.hw = NKV % 8 == 0 ? 8 : NKV % 4 == 0 ? 4 : NKV % 2 == 0 ? 2 : 1;
+  p.hw = heads_per_workgroup(NKV);
   p.ncg = p.mfma ? kCols : (NC < kGenOut / D ? NC : kGenOut / D);
   p.passes = (NC + p.ncg - 1) / p.ncg;
   p.ncp = p.passes * p.ncg;

@@ -1193,9 +1193,13 @@ def rope_cache(max_position: int, head_dim: int, theta: float, *,
     return torch.cos(angles).contiguous(), torch.sin(angles).contiguous()
 
 
-# (query, head of a group) columns up to which position-free pages are never staged
-# (window_pays in position_free.hip)
-POSITION_FREE_WALKED = 55
+
+def _may_stage_pages(cols: int, elems: int) -> bool:
+    """Whether a position-free call of so many (query, head of a group) columns over
+    so many elements of K may take the staged route: the weakest of kStageRules in
+    position_free.hip (fp32 pages and other head dims never do)."""
+    return cols >= 48 and (cols - 48) * elems >= 17 << 19
+
 
 DTYPE_CODES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}  # VOOM_DTYPE_*
 
@@ -1260,12 +1264,13 @@ def position_free_paged_attention(q: torch.Tensor, k_pages: torch.Tensor, v_page
                                   stream=stream)
     need = position_free_workspace_bytes(B, NQ, TQ, NKV, D, TK, q.dtype, num_splits)
     side = _side_stream(stream)
-    if side is not None or B * (NQ // NKV) * TQ > POSITION_FREE_WALKED:
-        # calls of many columns may keep a copy of the pages in their workspace
-        # (megabytes to a gigabyte): their own, given back when they have run, on
-        # the stream that uses it
-        with torch.cuda.stream(stream):
+    # A copy of the pages in the workspace (megabytes to a gigabyte) is the call's
+    # own, given back when it has run, and made on the stream that uses it.
+    if side is not None:
+        with torch.cuda.stream(side):
             ws = torch.empty(max(need, 256), dtype=torch.uint8, device=q.device)
+    elif _may_stage_pages(B * (NQ // NKV) * TQ, TK * NKV * D):
+        ws = torch.empty(max(need, 256), dtype=torch.uint8, device=q.device)
     else:
         ws = workspace(q.device, need, tag=3)
     out = torch.empty_like(q)
