@@ -145,6 +145,20 @@ def test_windows_equal_one_query_at_a_time(dtype):
         assert rel <= 2 * REL[dtype], (BLOCK, splits, scale, rel)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_nan_keys_stay_nan(dtype):
+    """Visible keys of NaN that fill whole splits (which then have no maximum) give
+    NaN in either route, and only for the heads that read them."""
+    print(f"[pf-window] NaN in K, {dtype}", flush=True)
+    for TQ, splits in ((3, 0), (3, 1), (3, 5), (staged_from(1, 8, 2, 64, 800), 0)):
+        args = list(inputs(1, 8, 2, TQ, 64, 1, 800, dtype, seed=3))
+        args[3] = torch.arange(800, dtype=torch.int32, device="cuda")
+        args[1][:300, 1] = float("nan")
+        out = ops.position_free_paged_attention(*args, scale=0.1, num_splits=splits)
+        torch.cuda.synchronize()
+        assert torch.isnan(out[0, 4:]).all() and torch.isfinite(out[0, :4]).all(), (TQ, splits)
+
+
 def test_weak_keys_keep_their_weight_in_fp16():
     """Weights far below fp16's normal range (2^-14 of the largest) still count:
     one key ahead of 4,000 others whose weights are 2^-16 of its own and whose

@@ -975,8 +975,8 @@ __global__ __launch_bounds__(kRedWaves * kWave) void pf_reduce_kernel(PfArgs a,
     acc = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int i = r; i < cnt; i += kRedRows) {
       const size_t p = (first + i) * a.NCP + n;
-      if (ml2[p].x != -INFINITY)
-        acc += *reinterpret_cast<const f32x4*>(a.part_o + p * D + dim0) * fast_exp2(ml2[p].x - M);
+      const float w = ml2[p].x == -INFINITY ? 0.f : fast_exp2(ml2[p].x - M);
+      acc += *reinterpret_cast<const f32x4*>(a.part_o + p * D + dim0) * w;
     }
   }
   // rows of one wave share M: the lanes of a column sum their rows
