@@ -86,6 +86,21 @@ def test_scales(scale):
     check(kv.attend_prefill(0, q, scale=scale), reference(q, k, v, scale))
 
 
+def test_a_scale_of_zero_keeps_nan():
+    """0 times an infinite or NaN query (or key) is NaN, as in the decode kernel;
+    other rows average the values they see."""
+    print("[prefill] scale 0, NaN in q and k", flush=True)
+    kv, q, k, v = build(1, 8, 2, 64, 64, 300, 40)
+    want = reference(q, k, v, 0.0)
+    q[0, 3, 7, 5], q[0, 6, 39, 63] = float("nan"), float("inf")
+    out = kv.attend_prefill(0, q, scale=0.0)
+    torch.cuda.synchronize()
+    hit = torch.zeros(out.shape[:3], dtype=torch.bool, device="cuda")
+    hit[0, 3, 7] = hit[0, 6, 39] = True
+    assert torch.isnan(out[hit]).all()
+    check(out.masked_fill(hit[..., None], 0.0), want.masked_fill(hit[..., None], 0.0))
+
+
 def test_rising_scores_move_the_reference_maximum():
     """Keys whose scores grow along the sequence: every tile's maximum is far
     above the last one's."""

@@ -34,6 +34,12 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, bf16x2_t));
 }
 
+// Two packed bf16 values times 0: NaN for an infinity or a NaN, else 0.
+__device__ __forceinline__ uint32_t nan_bf16(uint32_t x) {
+  return ((x & 0x7f80u) == 0x7f80u ? 0xffffu : 0u) |
+         ((x & 0x7f800000u) == 0x7f800000u ? 0xffff0000u : 0u);
+}
+
 // a.lo + a.hi (+ c) of two packed bf16 values in fp32: one v_dot2_f32_bf16
 // against (1, 1).
 __device__ __forceinline__ float sum_bf16x2(uint32_t a, float c) {

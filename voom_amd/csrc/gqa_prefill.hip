@@ -73,9 +73,11 @@ struct PrefillArgs {
   int per_xcd;    // work items per XCD
   int xcd_cus;    // CUs per XCD
   // |softmax scale| in log2 units, > 0.  The sign is applied to q (q_flip =
-  // 0x80008000), a scale of 0 by clearing q (q_keep = 0, scale 1).
+  // 0x80008000), a scale of 0 by clearing q but for infinities and NaN (q_zero,
+  // scale 1).
   float scale;
-  uint32_t q_keep, q_flip;
+  uint32_t q_flip;
+  bool q_zero;
 };
 
 // Key (0..31 of a block) that row r of the score tile holds: lane half h then
@@ -153,7 +155,14 @@ void gqa_prefill_kernel(PrefillArgs a) {
     for (int s = 0; s < KS; ++s) {
       qop[s] = *reinterpret_cast<const u32x4*>(qh + 16 * s);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) qop[s][i] = (qop[s][i] & a.q_keep) ^ a.q_flip;
+      for (int i = 0; i < 4; ++i) qop[s][i] ^= a.q_flip;
+    }
+    if (a.q_zero) {
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) qop[s][i] = nan_bf16(qop[s][i]);
+      }
     }
   };
 
@@ -671,7 +680,7 @@ extern "C" int voom_paged_gqa_prefill(const void* q, const void* k_pool, const v
   a.per_xcd = (a.work + 7) / 8;
   a.xcd_cus = device_cu_count() / 8;
   a.scale = scale == 0.f ? 1.f : fabsf(scale) * 1.4426950408889634f;
-  a.q_keep = scale == 0.f ? 0u : 0xffffffffu;
+  a.q_zero = scale == 0.f;
   a.q_flip = scale < 0.f ? 0x80008000u : 0u;
   const dim3 grid(static_cast<unsigned>(8 * a.per_xcd));
   const dim3 block(NW * kWave);
