@@ -167,8 +167,9 @@ inline int ilog2(long long x) {
 // Key splits of a window of `wgs` workgroups of equal rows (gqa_prefill.hip,
 // position_free.hip): as many as leave at most one workgroup per CU, since a CU
 // that gets two while others have one takes twice as long (56 workgroups, 126
-// tiles: five splits 94 us, four 82 us), unless a quarter of the CUs would idle
-// (160 workgroups, 82 tiles: one split 93 us, three 83 us); 1 from one per CU on.
+// tiles: five splits 94 us, four 82 us).  Where that is a single split with a
+// quarter of the CUs idle, as many as fill two rounds (160 workgroups, 82 tiles: one
+// split 93 us, three 83 us); 1 from one workgroup per CU on.
 inline long long key_splits(long long wgs, int cus) {
   if (wgs >= cus) return 1;
   const long long s = cus / wgs;

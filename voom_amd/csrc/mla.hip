@@ -1336,16 +1336,16 @@ __global__ __launch_bounds__(kRgWaves* kWave) void mla_reduce_groups_kernel(
   if (lse_out != nullptr && lane == 0) lse_out[task] = merged_lse(M, L);
 }
 
-// Merge and output projection fused, one workgroup per head (64-head-group
-// partials): weighted_c [b, h, :] for every sequence b, rounded to bf16 as the
+// Merge and output projection fused, two workgroups per head, each for half of its
+// column tiles (one workgroup where dv is a single tile; 64-head-group partials): weighted_c [b, h, :] for every sequence b, rounded to bf16 as the
 // reference rounds it (runtime/glm.py:162-164), then y [b, h, :dv] =
 // weighted_c . W_UV (runtime/glm.py:200-202) on v_mfma_f32_16x16x32_bf16 with
-// the sequences as the M = 16 dimension.  W_UV[h] (packed as for
-// voom_mla_head_gemv, dv <= 128: at most 128 KiB) streams into LDS from the
+// the sequences as the M = 16 dimension.  The workgroup's part of W_UV[h] (packed as
+// for voom_mla_head_gemv, dv <= 128: at most 64 KiB) streams into LDS from the
 // first instruction on, beside the partial rows the merge reads, so one
 // launch replaces the merge and the projection's weight stream.  Eight
 // wavefronts: wavefront w merges sequences w, w + 8 (or, with many ranges,
-// their groups of ranges), then projects column tiles w, w + 8.
+// their groups of ranges), then projects a column tile.
 constexpr int kRpMaxTiles = 8;                 // dv <= 128
 constexpr int kRpPartTiles = kRpMaxTiles / 2;  // column tiles of one workgroup (two parts)
 constexpr int kRpSteps = kC / kHgStep;         // 16 k-steps over the 512 latent dims
@@ -1452,8 +1452,9 @@ int default_ranges(int B, int H) {
   return nr < 1 ? 1 : nr;
 }
 
-// Ranges of a dense call over tables of at most `tiles` 64-token tiles: of the
-// counts that default_ranges allows, the one with the least of
+// Ranges of a dense call over tables of at most `tiles` 64-token tiles (the table's
+// capacity: the host does not know the contexts): of the counts that default_ranges
+// allows, the one with the least of
 //   1.75 us per tile of a range (they run one after the other),
 //   0.03 us per workgroup for its partial rows, written and read back,
 //   1 us per round trip of the grouped merge past 16 ranges, 0.25 us per range
@@ -1461,7 +1462,9 @@ int default_ranges(int B, int H) {
 // Fitted to sweeps over 1-16 sequences of 200-65,536 tokens and 32-128 heads;
 // default_ranges alone, before: 128 heads, 1 sequence of 200 / 1,000 / 16,384
 // tokens 36 / 35 / 38 us, now 20 / 20 / 29; 6 of 8,000: 51, now 39; 64 heads, 1 of
-// 1,000: 44, now 18.
+// 1,000: 44, now 18.  Those are tight tables; a table twice or eight times as wide as
+// its contexts gets a count meant for longer ones, which costs at most 3% against
+// default_ranges alone (32 heads, 8 of 4,000 in a table for 8,000: 21.4 and 22.1 us).
 int dense_ranges(int B, int H, long long tiles) {
   const int hg = heads_per_group(H);
   const int most = default_ranges(B, H);
@@ -1825,7 +1828,7 @@ int launch_head_rows(HeadRows a, hipStream_t stream) {
   a.NT = (a.N + kHgTile - 1) / kHgTile;
   a.KS = (a.K + kHgStep - 1) / kHgStep;
   a.groups = (a.rows + 15) / 16;
-  const int tpw = a.KS <= 4 ? 4 : a.KS <= 8 ? 4 : 2;
+  const int tpw = a.KS <= 8 ? 4 : 2;
   const int waves = kThreads / kWave;
   const int bx = (a.NT + waves * tpw - 1) / (waves * tpw);
   // about one workgroup per CU: the weights are read once per z, and a wavefront

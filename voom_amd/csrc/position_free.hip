@@ -1771,11 +1771,9 @@ int launch_pf_window(const PfPlan& p, const PfArgs& a, char* ws, bool f32_tab, v
   w.scale = a.scale == 0.f ? 1.f : fabsf(a.scale_log2e);
   w.q_keep = a.scale == 0.f ? 0u : 0xffffffffu;
   w.q_flip = a.scale < 0.f ? 0x80008000u : 0u;
-  if (p.nblk > 0) {
-    const dim3 grid(static_cast<unsigned>(p.nblk) * a.NKV);
-    if (f32_tab) hipLaunchKernelGGL((pf_stage_kernel<D, E, EF32>), grid, dim3(256), 0, stream, w);
-    else hipLaunchKernelGGL((pf_stage_kernel<D, E, E>), grid, dim3(256), 0, stream, w);
-  }
+  const dim3 grid(static_cast<unsigned>(p.nblk) * a.NKV);
+  if (f32_tab) hipLaunchKernelGGL((pf_stage_kernel<D, E, EF32>), grid, dim3(256), 0, stream, w);
+  else hipLaunchKernelGGL((pf_stage_kernel<D, E, E>), grid, dim3(256), 0, stream, w);
   hipLaunchKernelGGL((pf_window_kernel<D, E>), dim3(8u * static_cast<unsigned>(w.per_xcd)),
                      dim3(kWinWaves * kWave), 0, stream, w, static_cast<uint16_t*>(out));
   int rc = VOOM_LAUNCH_CHECK("position_free_attention: window launch");
