@@ -86,6 +86,24 @@ def test_scales(scale):
     check(kv.attend_prefill(0, q, scale=scale), reference(q, k, v, scale))
 
 
+@pytest.mark.parametrize("L,first,count", [(3, 64, 2900), (3, 2048, 700), (40, 512, 1600),
+                                           (700, 0, 200)])
+def test_keys_pushed_to_minus_infinity(L, first, count):
+    """Whole tiles of visible keys that score -inf weigh nothing, at the start of the
+    window and of a key split (3 queries: every fourth tile begins one) too."""
+    print(f"[prefill] -inf keys {first} + {count}, window {L}", flush=True)
+    S, D = 3000, 128
+    kv, q, k, v = build(1, 8, 2, D, 64, S, L)
+    k[:, :, first:first + count] = 0
+    k[:, :, first:first + count, 5] = torch.finfo(torch.bfloat16).min
+    q[..., 5] = 4.0  # 4 times the lowest value is past fp32's range
+    kv = PagedKVCache(1, 1 << 40, page_positions=64)
+    kv.append(0, k, v)
+    k64 = k.double()
+    k64[:, :, first:first + count, 5] = -float("inf")
+    check(kv.attend_prefill(0, q, scale=0.1), reference(q, k64, v, 0.1))
+
+
 def test_a_scale_of_zero_keeps_nan():
     """0 times an infinite or NaN query (or key) is NaN, as in the decode kernel;
     other rows average the values they see."""

@@ -42,6 +42,7 @@
 // splits leave (m, l, o) in fp32 and gqa_prefill_combine_kernel merges them.
 #include "common.h"
 
+#include <cfloat>
 #include <type_traits>
 
 namespace voom {
@@ -233,7 +234,9 @@ void gqa_prefill_kernel(PrefillArgs a) {
   f32x16 acc[DT];
 #pragma unroll
   for (int d = 0; d < DT; ++d) acc[d] = f32x16{};
-  float m = -INFINITY;  // reference maximum, log2 units; the same in both halves
+  // Reference maximum, log2 units; the same in both halves.  Never -inf: keys of
+  // score -inf (masked or not) then have P = 0 also where nothing else came before.
+  float m = -FLT_MAX;
   float l = 0.f;        // over this lane's keys
 
   typedef f32x16 Scores[2];  // 32-key blocks of a tile; accumulator i of block
@@ -260,7 +263,7 @@ void gqa_prefill_kernel(PrefillArgs a) {
     mx = fmaxf(mx, __shfl_xor(mx, 32)) * a.scale;
     if (__builtin_amdgcn_ballot_w64(mx > m) == 0) return;
     const float mn = fmaxf(m, mx);
-    float alpha = mn == -INFINITY ? 1.f : fast_exp2(m - mn);
+    float alpha = fast_exp2(m - mn);
     asm volatile("" : "+v"(alpha));
     m = mn;
     l *= alpha;
@@ -372,7 +375,7 @@ void gqa_prefill_kernel(PrefillArgs a) {
   // Any tile t that some row of the wavefront sees: its scores are in sc, which
   // then takes those of tile t + 1 if a row sees that too.
   auto edge_tile = [&](int t, const uint16_t* tile, Scores& sc) {
-    const float mref = m == -INFINITY ? 0.f : m;  // nothing visible yet: P = 0
+    const float mref = m;
     u32x4 pk[2][2];
 #pragma unroll
     for (int e = 0; e < 16; ++e) form_p(e, sc, mref, pk);
@@ -544,8 +547,8 @@ __global__ __launch_bounds__(kCombineWaves * kWave) void gqa_prefill_combine_ker
   const bool live = lane < a.splits;
   const float2 ml = ml2[p0 + (live ? lane : 0)];
   const float M = wave_max_uniform(live ? ml.x : -INFINITY);
-  // a split that holds no visible key of the row left m = -inf, l = 0
-  const float wt = live && ml.x != -INFINITY ? fast_exp2(ml.x - M) : 0.f;
+  // (a split that holds no visible key of the row left m = -FLT_MAX, l = 0)
+  const float wt = live ? fast_exp2(ml.x - M) : 0.f;
   const float inv = 1.f / wave_sum_uniform(live ? ml.y * wt : 0.f);
   float acc[DPL] = {};
   const float* po = a.part_o + p0 * D + lane * DPL;
