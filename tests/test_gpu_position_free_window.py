@@ -325,3 +325,27 @@ def test_windows_on_a_side_stream():
         del junk
         torch.cuda.synchronize()
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+def test_captured_windows_replay():
+    """A captured window keeps its workspace: replays between eager calls of larger
+    windows equal the eager result."""
+    print("[pf-window] graph replay", flush=True)
+    args = inputs(1, 28, 4, 100, 128, 1, 3000, torch.float16, seed=4)
+    other = inputs(1, 28, 4, 250, 128, 1, 8000, torch.bfloat16, seed=5)
+    want = ops.position_free_paged_attention(*args, scale=0.1)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(graph, stream=side):
+            out = ops.position_free_paged_attention(*args, scale=0.1)
+    torch.cuda.current_stream().wait_stream(side)
+    for _ in range(3):
+        out.zero_()
+        ops.position_free_paged_attention(*other, scale=0.1)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16))

@@ -43,6 +43,7 @@
 // so P^T is used straight from the score registers.
 #include "common.h"
 
+#include <float.h>
 #include <limits.h>
 
 namespace voom {
@@ -1314,7 +1315,8 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
   f32x16 acc[DT];
 #pragma unroll
   for (int d = 0; d < DT; ++d) acc[d] = f32x16{};
-  float m = -INFINITY;
+  // never -inf, as in gqa_prefill_kernel: keys of score -inf have P = 0
+  float m = -FLT_MAX;
   float l = 0.f;
 
   typedef f32x16 Scores[2];  // accumulator i of block j: key 32 j + 16 (i / 8) + 8 lh + i % 8
@@ -1343,7 +1345,7 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
     mx = fmaxf(mx, __shfl_xor(mx, 32)) * wa.scale;
     if (__builtin_amdgcn_ballot_w64(mx > m) == 0) return;
     const float mn = fmaxf(m, mx);
-    float alpha = mn == -INFINITY ? 1.f : fast_exp2(m - mn);
+    float alpha = fast_exp2(m - mn);
     asm volatile("" : "+v"(alpha));  // keeps the rescaling inside the branch
     m = mn;
     l *= alpha;
@@ -1380,7 +1382,7 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
   // Tile t where every row of the wavefront sees all of tiles t and t + 1.
   auto whole_tile = [&](int t, const uint16_t* tile, uint16_t* next, const Scores& sc,
                         Scores& nx) {
-    const float mref = m == -INFINITY ? 0.f : m;  // every key so far scored -inf: P = 0
+    const float mref = m;
     Weights pk;
     u32x4 ring[kA];
 #pragma unroll
@@ -1436,7 +1438,7 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
   // Any tile t: its scores are in sc, which then takes those of tile t + 1.
   auto edge_tile = [&](int t, const uint16_t* tile, Scores& sc) {
     if (seen(t)) {
-      const float mref = m == -INFINITY ? 0.f : m;  // nothing visible yet: P = 0
+      const float mref = m;
       Weights pk;
 #pragma unroll
       for (int e = 0; e < 16; ++e) form_p(e, sc, mref, pk);
@@ -1482,8 +1484,7 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
       }
     }
     s += __shfl_xor(s, 32);
-    const float ref = m == -INFINITY ? 0.f : m;
-    const float wt = whole_weight(fast_exp2(__builtin_fmaf(s, wa.scale, -ref)));
+    const float wt = whole_weight(fast_exp2(__builtin_fmaf(s, wa.scale, -m)));
     const bool sees = wa.pos[kt] <= qpos;
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
@@ -1599,8 +1600,8 @@ __global__ __launch_bounds__(256) void pf_window_combine_kernel(WinArgs wa, uint
   const bool live = lane < wa.splits;
   const float2 ml = reinterpret_cast<const float2*>(a.part_ml)[p0 + (live ? lane : 0)];
   const float M = wave_max_uniform(live ? ml.x : -INFINITY);
-  // a split that holds no visible key of the row left m = -inf, l = 0
-  const float wt = live && ml.x != -INFINITY ? fast_exp2(ml.x - M) : 0.f;
+  // (a split that holds no visible key of the row left m = -FLT_MAX, l = 0)
+  const float wt = live ? fast_exp2(ml.x - M) : 0.f;
   const float lt = wave_sum_uniform(live ? ml.y * wt : 0.f);
   const int c = lane % kLanes, side = lane / kLanes;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
