@@ -1027,8 +1027,8 @@ __global__ __launch_bounds__(kRedWaves * kWave) void pf_reduce_kernel(PfArgs a,
 // scores^T and out^T on 32x32x16 MFMAs, P^T in registers, the scores one tile
 // ahead of P . V, operands straight into LDS, one barrier per tile.  250 queries
 // over 8,003 keys (28q/4kv, D = 128): fp16 3,866 us in the generic kernel, 446 in
-// pf_attention_kernel's 110 passes, 78 here (11 staging, 60 the window kernel, 5
-// the merge of its splits); bf16 449 and 65 us.
+// pf_attention_kernel's 110 passes, 72 here (11 of them staging, 5 the merge of its
+// splits); bf16 449 and 60 us.
 constexpr int kWinWaves = 4;
 constexpr int kWinRows = 32;                       // rows of a wavefront
 constexpr int kWinTile = kWinWaves * kWinRows;     // rows of a workgroup
