@@ -611,7 +611,8 @@ void pf_attention_kernel(PfArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) any = __builtin_fmaf(acc[d][r], 0.f, any);
     }
-    if (__builtin_amdgcn_ballot_w64(any != 0.f) != 0) {
+    // (a NaN among the weights makes the whole row NaN: nothing to look for)
+    if (__builtin_amdgcn_ballot_w64(any != 0.f && l_lane * 0.f == 0.f) != 0) {
       f32x4 odd[DT] = {};
       for (int key = blo * kKeys; key < min(bhi * kKeys, a.TK); ++key) {
         int pg, ps, rlo, rhi, kp;
