@@ -85,7 +85,8 @@ def staged_from(B, NQ, NKV, D, TK):
 def test_staged_from_is_the_rule():
     """The workspace tells the routes apart: partials of many splits against the
     staged pages."""
-    for B, NQ, NKV, D, TK in ((1, 28, 4, 128, 3000), (1, 32, 8, 128, 700), (1, 8, 8, 128, 9000), (2, 9, 3, 64, 5000),
+    for B, NQ, NKV, D, TK in ((1, 28, 4, 128, 3000), (1, 32, 8, 128, 700), (1, 8, 8, 128, 9000),
+                              (2, 9, 3, 64, 5000),
                               (1, 4, 2, 64, 8000), (1, 16, 2, 128, 900), (1, 8, 8, 64, 2000),
                               (1, 12, 12, 64, 1500), (1, 7, 1, 128, 20000)):
         TQ = staged_from(B, NQ, NKV, D, TK)
@@ -271,9 +272,9 @@ def test_infinite_values_of_one_head(NQ, NKV, D, TK):
 
 @pytest.mark.parametrize("wide", [False, True])
 def test_weights_of_fp16_pages_to_32_bits(wide):
-    """Two keys of a block with values +-2^15 whose weights differ by d = 2^-15 .. 2^-13 (all
-    others weigh nothing) leave 2^15 tanh(d / 2): what the weights' own rounding adds is not hidden by the
-    output's.  Bound, for the weight just below 1: the exponential 2^-24 (an ulp),
+    """Two keys of a block with values +-2^15 whose weights differ by d = 2^-15 ..
+    2^-13 (all others weigh nothing) leave 2^15 tanh(d / 2): what the weights' own
+    rounding adds is not hidden by the output's.  Bound, for the weight just below 1: the exponential 2^-24 (an ulp),
     hi and lo halves 2^-24, the sums behind them as much again, times 2^14; fp16
     output 2^-12 of the value; scores of this size are exact to 2^-37."""
     TK = 4000

@@ -1337,7 +1337,8 @@ __global__ __launch_bounds__(kRgWaves* kWave) void mla_reduce_groups_kernel(
 }
 
 // Merge and output projection fused, two workgroups per head, each for half of its
-// column tiles (one workgroup where dv is a single tile; 64-head-group partials): weighted_c [b, h, :] for every sequence b, rounded to bf16 as the
+// column tiles (one workgroup where dv is a single tile; 64-head-group partials):
+// weighted_c [b, h, :] for every sequence b, rounded to bf16 as the
 // reference rounds it (runtime/glm.py:162-164), then y [b, h, :dv] =
 // weighted_c . W_UV (runtime/glm.py:200-202) on v_mfma_f32_16x16x32_bf16 with
 // the sequences as the M = 16 dimension.  The workgroup's part of W_UV[h] (packed as

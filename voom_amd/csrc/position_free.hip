@@ -1467,8 +1467,8 @@ void pf_window_kernel(WinArgs wa, uint16_t* out) {
     const int tb = kt / a.BLOCK;
     int page = a.table[tb];
     page = static_cast<unsigned>(page) < static_cast<unsigned>(a.P) ? page : 0;
-    const uint16_t* vr = static_cast<const uint16_t*>(a.v_pages) +
-                         ((static_cast<size_t>(page) * a.NKV + kvh) * a.BLOCK + (kt - tb * a.BLOCK)) * D;
+    const size_t row = (static_cast<size_t>(page) * a.NKV + kvh) * a.BLOCK + (kt - tb * a.BLOCK);
+    const uint16_t* vr = static_cast<const uint16_t*>(a.v_pages) + row * D;
     uint32_t any = 0;
 #pragma unroll
     for (int i = 0; i < D / kWave; ++i) any |= odd_halves(vr[i * kWave + lane]);
